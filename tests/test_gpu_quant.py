@@ -121,6 +121,33 @@ def test_quantize_mixed_zero_minima(K, N, G, dtype):
         assert (zb == 0x8000).any() and (zb == 0x0000).any()   # both zero signs occur
 
 
+@pytest.mark.parametrize("N", [260, 261])
+@pytest.mark.parametrize("G", [8, 16, 24, 32, 40, 64, 72, 96, 128, 136, 256, 264, 520])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_quantize_ties_and_scales_every_group_split(G, dtype, N):
+    """Every split of a group over waves and registers (one, two or four waves a
+    group, one to eight packed rows a wave, long groups read twice), an odd
+    number of groups and a partial column block (N % 4 == 0 and not), on columns
+    whose quotients lie on or one ulp beside a rounding tie, whose scales are
+    powers of two, or whose scales lie outside the range of the
+    corrected-reciprocal quotient (fp32)."""
+    log(f"quantize ties G={G} N={N} {dtype}")
+    K = 5 * G
+    rng = np.random.default_rng(G * 2 + N % 4)
+    t = rng.integers(0, 16, (K, N)) + rng.choice([0.0, 0.5], (K, N))
+    s = np.exp2(rng.integers(-6, 1, N)) * rng.choice([1.0, 1.0, 1.1, 1.37], N)
+    W = ((np.minimum(t, 15.0) - rng.integers(0, 16, N)) * s).astype(np.float32)
+    W[::G], W[1::G] = W.min(axis=0), W.min(axis=0) + 15 * s.astype(np.float32)
+    if dtype == torch.float32:
+        step = rng.integers(-1, 2, W.shape)
+        beside = np.nextafter(W, np.where(step > 0, np.inf, -np.inf), dtype=np.float32)
+        W = np.where(step == 0, W, beside)
+        W[:, 64:68] *= np.float32(2.0 ** -110)
+        W[:, 128:132] *= np.float32(2.0 ** 118)
+        W[:, 200:204] += np.float32(1000.0)
+    _assert_quant_equal(torch.from_numpy(W).to(dtype), G, f"ties G={G} N={N}")
+
+
 def test_quantize_fp32_tiny_and_denormal_ranges():
     log("quantize fp32 tiny ranges")
     K, N, G = 64, 8, 32

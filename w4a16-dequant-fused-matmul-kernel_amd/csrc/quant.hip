@@ -24,6 +24,8 @@
 #include "w4a16_device.h"
 #include "w4a16_launch.h"
 
+#include <type_traits>
+
 namespace w4a16 {
 namespace {
 
@@ -32,28 +34,12 @@ struct InF16 {
   typedef uint16_t T;
   static __device__ __forceinline__ float val(T b) { return (float)as_h(b); }
   static __device__ __forceinline__ bool nonfinite(T b) { return (b & 0x7C00u) == 0x7C00u; }
-  // four consecutive elements (8-byte aligned)
-  static __device__ __forceinline__ void load4(const T* p, T out[4]) {
-    const uint2 v = *reinterpret_cast<const uint2*>(p);
-    out[0] = v.x & 0xFFFFu;
-    out[1] = v.x >> 16;
-    out[2] = v.y & 0xFFFFu;
-    out[3] = v.y >> 16;
-  }
 };
 struct InF32 {
   typedef float T;
   static __device__ __forceinline__ float val(T v) { return v; }
   static __device__ __forceinline__ bool nonfinite(T v) {
     return (__builtin_bit_cast(uint32_t, v) & 0x7F800000u) == 0x7F800000u;
-  }
-  // four consecutive elements (16-byte aligned)
-  static __device__ __forceinline__ void load4(const T* p, T out[4]) {
-    const float4 v = *reinterpret_cast<const float4*>(p);
-    out[0] = v.x;
-    out[1] = v.y;
-    out[2] = v.z;
-    out[3] = v.w;
   }
 };
 
@@ -100,242 +86,318 @@ __device__ __forceinline__ float clamp_q(float v) {
   return v;
 }
 
-template <class IN, int CPT>
-__device__ __forceinline__ void load_row(const typename IN::T* p, typename IN::T b[CPT]) {
-  if constexpr (CPT == 4) {
-    IN::load4(p, b);
+// One group's column: fp32 scale s, r = the rounded 1 / s, zero-point z.
+struct QCol {
+  float s, r, z;
+};
+
+__device__ __forceinline__ QCol make_qcol(float mn, float mx) {
+  QCol c;
+  const float s = (mx - mn) / 15.0f;
+  c.s = (s > 0.0f) ? s : 1.0f;
+  c.r = 1.0f / c.s;
+  c.z = clamp_q(__builtin_rintf(-mn / c.s));
+  return c;
+}
+
+// Scales for which code_of's five-operation quotient is the IEEE one wherever
+// its rounding can matter (|v / s| >= 1/4): there the reciprocal is normal and
+// the residual v - q s, a multiple of 2^-48 s / 4, is not below the smallest
+// subnormal.
+__device__ __forceinline__ bool fast_scale(float s) { return s >= 0x1p-96f && s <= 0x1p120f; }
+
+// clamp(rint(v / s) + z, 0, 15) as a whole float.  kDiv: by IEEE division,
+// about ten instructions a weight, which bound the kernel (VALU-bound at 2.5
+// TB/s of an achievable 5.1).  Else by Markstein's correction (P. Markstein,
+// "Computation of elementary functions on the IBM RISC System/6000 processor",
+// 1990): with r = RN(1 / s), one step from v r gives a faithful quotient and a
+// second the correctly rounded one.  An fp16 v enters the fused operations
+// unconverted (v_fma_mix_f32).
+template <bool kDiv, class H>
+__device__ __forceinline__ float code_of(H v, const QCol& c) {
+  float q;
+  if constexpr (kDiv) {
+    q = (float)v / c.s;
   } else {
-#pragma unroll
-    for (int c = 0; c < CPT; ++c) b[c] = p[c];
+    q = __builtin_fmaf((float)v, c.r, 0.0f);
+    q = __builtin_fmaf(__builtin_fmaf(-q, c.s, (float)v), c.r, q);
+    q = __builtin_fmaf(__builtin_fmaf(-q, c.s, (float)v), c.r, q);
   }
+  return __builtin_amdgcn_fmed3f(__builtin_rintf(q) + c.z, 0.0f, 15.0f);
 }
 
-// One thread quantises CPT adjacent columns of one group (G % 8 == 0).
-template <class IN, int CPT>
-__global__ __launch_bounds__(256) void quantize_kernel(const typename IN::T* __restrict__ W,
-                                                       uint32_t* __restrict__ QW,
-                                                       uint16_t* __restrict__ SC,
-                                                       uint16_t* __restrict__ ZR, int K, int N,
-                                                       int G, int32_t* __restrict__ flag) {
-  typedef typename IN::T T;
-  const int n = (blockIdx.y * 256 + threadIdx.x) * CPT;
-  const int g = blockIdx.x;
-  if (n >= N) return;
-  const T* src = W + (size_t)g * G * N + n;
-  // CPT divides 32 and n is a multiple of CPT: all CPT columns lie on one side.
-  static_assert(32 % CPT == 0, "a thread's columns must not straddle a 32-column block");
-  const bool tie_last = n < 32 * (N / 32);
-
-  float mn[CPT], mx[CPT];
-  bool bad = false;
-  {
-    T b[CPT];
-    load_row<IN, CPT>(src, b);
+// Eight codes (whole floats in [0, 15], row order) to a packed word: two exact
+// sums below 2^16.
+__device__ __forceinline__ uint32_t pack_codes(const float q[8]) {
+  uint32_t half[2];
 #pragma unroll
-    for (int c = 0; c < CPT; ++c) {
-      bad |= IN::nonfinite(b[c]);
-      mn[c] = mx[c] = IN::val(b[c]);
-    }
-  }
-  for (int r = 1; r < G; ++r) {
-    T b[CPT];
-    load_row<IN, CPT>(src + (size_t)r * N, b);
-#pragma unroll
-    for (int c = 0; c < CPT; ++c) {
-      bad |= IN::nonfinite(b[c]);
-      const float v = IN::val(b[c]);
-      mn[c] = min_step(v, mn[c], tie_last);
-      mx[c] = (v >= mx[c]) ? v : mx[c];
-    }
-  }
-  if (bad) *flag = 1;
-  if constexpr (CPT == 1) {
-    if (N == 1 && G >= 32 && mn[0] == 0.0f) mn[0] = inner_zero_min<IN>(src, G);
-  }
-
-  float sc[CPT], zr[CPT];
-#pragma unroll
-  for (int c = 0; c < CPT; ++c) {
-    float s = (mx[c] - mn[c]) / 15.0f;
-    s = (s > 0.0f) ? s : 1.0f;
-    sc[c] = s;
-    zr[c] = clamp_q(__builtin_rintf(-mn[c] / s));
-  }
-
-  for (int r8 = 0; r8 < G / 8; ++r8) {
-    uint32_t word[CPT];
-#pragma unroll
-    for (int c = 0; c < CPT; ++c) word[c] = 0u;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      T b[CPT];
-      load_row<IN, CPT>(src + (size_t)(r8 * 8 + j) * N, b);
-#pragma unroll
-      for (int c = 0; c < CPT; ++c) {
-        const float q = clamp_q(__builtin_rintf(IN::val(b[c]) / sc[c]) + zr[c]);
-        word[c] |= ((uint32_t)(int)q & 0xFu) << (4 * j);
-      }
-    }
-    uint32_t* dst = QW + (size_t)(g * (G / 8) + r8) * N + n;
-    if constexpr (CPT == 4) {
-      *reinterpret_cast<uint4*>(dst) = make_uint4(word[0], word[1], word[2], word[3]);
-    } else {
-#pragma unroll
-      for (int c = 0; c < CPT; ++c) dst[c] = word[c];
-    }
-  }
-#pragma unroll
-  for (int c = 0; c < CPT; ++c) {
-    SC[(size_t)g * N + n + c] = as_u16((f16)sc[c]);
-    ZR[(size_t)g * N + n + c] = as_u16((f16)zr[c]);
-  }
+  for (int h = 0; h < 2; ++h)
+    half[h] = (uint32_t)__builtin_fmaf(
+        q[4 * h + 3], 4096.0f,
+        __builtin_fmaf(q[4 * h + 2], 256.0f, __builtin_fmaf(q[4 * h + 1], 16.0f, q[4 * h])));
+  return half[0] | (half[1] << 16);
 }
 
-// Four adjacent columns' weights of one row: 8 (fp16) or 16 (fp32) bytes.
+// Four columns' weights of one row, and their running minimum and maximum: four
+// adjacent columns in one load of 8 (fp16) or 16 (fp32) bytes, or columns 64
+// apart (`left` of them inside N, in each lane's order) in one load each.  minimum / maximum here are the IEEE 754
+// ones (v_pk_minimum3_f16, v_minimum3_f32: two rows per instruction, for fp16
+// of two columns): a NaN in any row survives to the end, and of two zeros the
+// minimum is -0 whatever their order, so a zero minimum's sign is found again
+// in row order (min_step).
 template <class IN>
 struct Row4;
 template <>
 struct Row4<InF16> {
+  typedef f16 H;
   uint2 v;
   __device__ __forceinline__ void load(const uint16_t* p) { v = *reinterpret_cast<const uint2*>(p); }
-  __device__ __forceinline__ uint16_t bits(int c) const {
-    return (uint16_t)(((c < 2 ? v.x : v.y) >> (16 * (c & 1))) & 0xFFFFu);
+  __device__ __forceinline__ void load_apart(const uint16_t* p, int left) {
+    const uint32_t a = left > 0 ? p[0] : 0u, b = left > 1 ? p[64] : 0u;
+    const uint32_t c = left > 2 ? p[128] : 0u, d = left > 3 ? p[192] : 0u;
+    v = make_uint2(a | (b << 16), c | (d << 16));
   }
-  __device__ __forceinline__ float val(int c) const { return InF16::val(bits(c)); }
-  __device__ __forceinline__ bool nonfinite(int c) const { return InF16::nonfinite(bits(c)); }
+  __device__ __forceinline__ H at(int c) const {
+    const f16x2 h = as_h2(c < 2 ? v.x : v.y);
+    return c & 1 ? h.y : h.x;
+  }
 };
 template <>
 struct Row4<InF32> {
+  typedef float H;
   float4 v;
   __device__ __forceinline__ void load(const float* p) { v = *reinterpret_cast<const float4*>(p); }
-  __device__ __forceinline__ float val(int c) const {
+  __device__ __forceinline__ void load_apart(const float* p, int left) {
+    v = make_float4(left > 0 ? p[0] : 0.0f, left > 1 ? p[64] : 0.0f, left > 2 ? p[128] : 0.0f,
+                    left > 3 ? p[192] : 0.0f);
+  }
+  __device__ __forceinline__ H at(int c) const {
     return c == 0 ? v.x : c == 1 ? v.y : c == 2 ? v.z : v.w;
   }
-  __device__ __forceinline__ bool nonfinite(int c) const { return InF32::nonfinite(val(c)); }
+};
+template <class IN>
+struct MinMax4;
+template <>
+struct MinMax4<InF16> {
+  f16x2 mn[2], mx[2];
+  __device__ __forceinline__ void first(const Row4<InF16>& r) {
+    mn[0] = mx[0] = as_h2(r.v.x);
+    mn[1] = mx[1] = as_h2(r.v.y);
+  }
+  __device__ __forceinline__ void add(const Row4<InF16>& r) {
+    const f16x2 h[2] = {as_h2(r.v.x), as_h2(r.v.y)};
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      mn[i] = __builtin_elementwise_minimum(mn[i], h[i]);
+      mx[i] = __builtin_elementwise_maximum(mx[i], h[i]);
+    }
+  }
+  __device__ __forceinline__ float lo(int c) const {
+    return (float)(c & 1 ? mn[c >> 1].y : mn[c >> 1].x);
+  }
+  __device__ __forceinline__ float hi(int c) const {
+    return (float)(c & 1 ? mx[c >> 1].y : mx[c >> 1].x);
+  }
+};
+template <>
+struct MinMax4<InF32> {
+  float mn[4], mx[4];
+  __device__ __forceinline__ void first(const Row4<InF32>& r) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) mn[c] = mx[c] = r.at(c);
+  }
+  __device__ __forceinline__ void add(const Row4<InF32>& r) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      mn[c] = __builtin_elementwise_minimum(mn[c], r.at(c));
+      mx[c] = __builtin_elementwise_maximum(mx[c], r.at(c));
+    }
+  }
+  __device__ __forceinline__ float lo(int c) const { return mn[c]; }
+  __device__ __forceinline__ float hi(int c) const { return mx[c]; }
 };
 
-// One workgroup quantises one group (G rows, G % 8 == 0) of 256 columns
-// (N % 4 == 0): lane l of each wave owns columns 4l..4l+3, and wave w a
-// contiguous quarter of the group's packed rows (octets).  Every lane issues
-// all of its rows' loads at once (the group's min / max no longer waits for
-// one row after another), the waves' minima and maxima meet in LDS in wave
-// (k) order, and the codes come from the rows still in registers (OPW > 0:
-// at most OPW octets per wave) or from a second read of the group (OPW = 0,
-// long groups; the tile is L2-resident).  The running minimum's tie rule
-// (min_step) applied within a wave in k order and across the waves in k order
-// gives the same zero as one scan in k order.  Grid: K / G x N / 256
-// workgroups (512 at K = N = 4096, G = 128, against 128 for one thread per
-// group and 4 columns).
-template <class IN, int OPW>
+__device__ __forceinline__ bool finite(float v) { return __builtin_fabsf(v) < __builtin_inff(); }
+
+// One workgroup of 4 waves quantises 4 / WPG groups (G rows, G % 8 == 0) of 256
+// columns: lane l of each wave owns columns 4l..4l+3 (VEC: N % 4 == 0 and
+// aligned W and qweight) or l, l + 64, l + 128, l + 192, and the WPG waves of a
+// group contiguous parts of its packed rows (octets), in k order.
+// Every lane issues all of its rows' loads at once, the minima and maxima of a
+// group's waves meet in LDS in wave (k) order, and the codes come from the rows
+// still in registers (OPW > 0: at most OPW octets per wave) or from a second
+// read of the group (OPW = 0, long groups; the tile is L2-resident).  The
+// running minimum's tie rule (min_step) applied within a wave in k order and
+// across the waves in k order gives the same zero as one scan in k order.
+// Column blocks are the fast grid index: neighbouring workgroups read
+// neighbouring 512-byte (fp16) pieces of the same rows.
+//
+// Bound by memory: about ten VALU instructions a weight, where an IEEE division
+// and an fp32 comparison per weight (about 34) had made it VALU-bound.  Measured
+// on MI355X, K = 4096, N = 14336, us: fp16 G = 128 / 64 / 32 61.2 / 55.7 / 55.3
+// -> 34.0 / 32.9 / 32.8 (4.4-4.7 TB/s of W read and the outputs written; a large
+// copy reaches 5.1), G = 4096 381 -> 171, fp32 G = 128 / 32 68.3 / 53.7 -> 47.4 /
+// 45.9; K = 8192, N = 28672 197 -> 115 (5.2 TB/s); N = 1001 (one thread per
+// column before) 30.8 -> 18.9.
+template <class IN, int OPW, int WPG, bool VEC>
 __global__ __launch_bounds__(256) void quantize_tile_kernel(const typename IN::T* __restrict__ W,
                                                             uint32_t* __restrict__ QW,
                                                             uint16_t* __restrict__ SC,
                                                             uint16_t* __restrict__ ZR, int K,
                                                             int N, int G,
                                                             int32_t* __restrict__ flag) {
-  __shared__ float smn[4][256], smx[4][256];
+  static_assert(WPG == 4 || (OPW > 0 && (WPG == 1 || WPG == 2)), "waves per group");
+  constexpr int GPB = 4 / WPG;   // groups per workgroup
+  __shared__ float smn[WPG > 1 ? 4 : 1][256], smx[WPG > 1 ? 4 : 1][256];
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
-  const int g = blockIdx.x;
-  const int n = blockIdx.y * 256 + 4 * lane;
-  const bool nv = n < N;
+  const int nblk = (N + 255) / 256;
+  const int g = (int)(blockIdx.x / (unsigned)nblk) * GPB + wave / WPG;
+  constexpr int kStep = VEC ? 1 : 64;   // between a lane's columns
+  const int n = (int)(blockIdx.x % (unsigned)nblk) * 256 + (VEC ? 4 : 1) * lane;
+  const int left = VEC ? 4 : (N - n + 63) / 64;   // of them inside N
   const int octs = G / 8;
-  const int per = (octs + 3) / 4;
-  const int o0 = min(octs, wave * per), o1 = min(octs, o0 + per);
-  const bool tie_last = n < 32 * (N / 32);
+  const int part = wave % WPG;
+  const int per = (octs + WPG - 1) / WPG;
+  const int o0 = min(octs, part * per), o1 = min(octs, o0 + per);
+  const bool nv = n < N && g < K / G;
+  bool tie_last[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) tie_last[c] = n + c * kStep < 32 * (N / 32);
   const typename IN::T* src = W + (size_t)g * G * N + n;
 
+  MinMax4<IN> mm;
   float mn[4], mx[4];
 #pragma unroll
   for (int c = 0; c < 4; ++c) {
     mn[c] = __builtin_inff();
     mx[c] = -__builtin_inff();
   }
-  bool bad = false;
-  auto scan = [&](const Row4<IN>& r) {
+  Row4<IN> keep[OPW > 0 ? OPW : 1][8];
+  auto load8 = [&](Row4<IN>(&r)[8], int o) {
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      bad |= r.nonfinite(c);
-      const float v = r.val(c);
-      mn[c] = min_step(v, mn[c], tie_last);
-      mx[c] = (v >= mx[c]) ? v : mx[c];
+    for (int j = 0; j < 8; ++j) {
+      const typename IN::T* p = src + (size_t)(o * 8 + j) * N;
+      if constexpr (VEC) r[j].load(p);
+      else r[j].load_apart(p, left);
     }
   };
-  Row4<IN> keep[OPW > 0 ? OPW : 1][8];
   if constexpr (OPW > 0) {
 #pragma unroll
     for (int i = 0; i < OPW; ++i)
-      if (nv && o0 + i < o1) {
+      if (nv && o0 + i < o1) load8(keep[i], o0 + i);
+  }
+  if (nv && o0 < o1) {
+    auto each = [&](auto&& f) {
+      if constexpr (OPW > 0) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) keep[i][j].load(src + (size_t)((o0 + i) * 8 + j) * N);
+        for (int i = 0; i < OPW; ++i)
+          if (o0 + i < o1) f(keep[i], i == 0);
+      } else {
+        for (int o = o0; o < o1; ++o) {
+          load8(keep[0], o);
+          f(keep[0], o == o0);
+        }
       }
+    };
+    each([&](const Row4<IN>(&r)[8], bool head) {
+      if (head) mm.first(r[0]);
+      else mm.add(r[0]);
 #pragma unroll
-    for (int i = 0; i < OPW; ++i)
-      if (nv && o0 + i < o1) {
+      for (int j = 1; j < 8; ++j) mm.add(r[j]);
+    });
+    bool bad = false, zero = false;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) scan(keep[i][j]);
-      }
-  } else if (nv) {
-    for (int o = o0; o < o1; ++o) {
-      Row4<IN> r[8];
+    for (int c = 0; c < 4; ++c) {
+      mn[c] = mm.lo(c);
+      mx[c] = mm.hi(c);
+      bad |= !finite(mn[c]) || !finite(mx[c]);
+      zero |= mn[c] == 0.0f;
+    }
+    if (bad) *flag = 1;
+    if (zero) {   // the sign of a zero minimum: the first or the last zero in k order
+      float z[4] = {__builtin_inff(), __builtin_inff(), __builtin_inff(), __builtin_inff()};
+      each([&](const Row4<IN>(&r)[8], bool) {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) r[j].load(src + (size_t)(o * 8 + j) * N);
+        for (int j = 0; j < 8; ++j)
 #pragma unroll
-      for (int j = 0; j < 8; ++j) scan(r[j]);
+          for (int c = 0; c < 4; ++c) z[c] = min_step((float)r[j].at(c), z[c], tie_last[c]);
+      });
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        if (mn[c] == 0.0f) mn[c] = z[c];
     }
   }
-  if (bad) *flag = 1;
+  if constexpr (WPG > 1) {
 #pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    smn[wave][4 * lane + c] = mn[c];
-    smx[wave][4 * lane + c] = mx[c];
-  }
-  __syncthreads();
-  float sc[4], zr[4];
-#pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    float a = smn[0][4 * lane + c], b = smx[0][4 * lane + c];
-#pragma unroll
-    for (int w = 1; w < 4; ++w) {
-      const float v = smn[w][4 * lane + c], u = smx[w][4 * lane + c];
-      a = min_step(v, a, tie_last);
-      b = (u >= b) ? u : b;
+    for (int c = 0; c < 4; ++c) {
+      smn[wave][4 * lane + c] = mn[c];
+      smx[wave][4 * lane + c] = mx[c];
     }
-    float s = (b - a) / 15.0f;
-    s = (s > 0.0f) ? s : 1.0f;
-    sc[c] = s;
-    zr[c] = clamp_q(__builtin_rintf(-a / s));
+    __syncthreads();
+    const int w0 = wave - part;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      mn[c] = smn[w0][4 * lane + c];
+      mx[c] = smx[w0][4 * lane + c];
+#pragma unroll
+      for (int w = 1; w < WPG; ++w) {
+        const float u = smx[w0 + w][4 * lane + c];
+        mn[c] = min_step(smn[w0 + w][4 * lane + c], mn[c], tie_last[c]);
+        mx[c] = (u >= mx[c]) ? u : mx[c];
+      }
+    }
   }
   if (!nv) return;
-  auto codes = [&](const Row4<IN>(&r)[8], int o) {
-    uint32_t word[4] = {0u, 0u, 0u, 0u};
-#pragma unroll
-    for (int j = 0; j < 8; ++j)
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const float q = clamp_q(__builtin_rintf(r[j].val(c) / sc[c]) + zr[c]);
-        word[c] |= ((uint32_t)(int)q & 0xFu) << (4 * j);
-      }
-    *reinterpret_cast<uint4*>(QW + (size_t)(g * octs + o) * N + n) =
-        make_uint4(word[0], word[1], word[2], word[3]);
-  };
-  if constexpr (OPW > 0) {
-#pragma unroll
-    for (int i = 0; i < OPW; ++i)
-      if (o0 + i < o1) codes(keep[i], o0 + i);
-  } else {
-    for (int o = o0; o < o1; ++o) {
-      Row4<IN> r[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) r[j].load(src + (size_t)(o * 8 + j) * N);
-      codes(r, o);
-    }
+  if constexpr (!VEC) {
+    if (N == 1 && G >= 32 && mn[0] == 0.0f) mn[0] = inner_zero_min<IN>(src, G);
   }
-  if (wave == 0) {
+  QCol qc[4];
+  bool fast = true;
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    qc[c] = make_qcol(mn[c], mx[c]);
+    fast &= fast_scale(qc[c].s);
+  }
+  auto codes = [&](auto div, const Row4<IN>(&r)[8], int o) {
+    uint32_t word[4];
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
-      SC[(size_t)g * N + n + c] = as_u16((f16)sc[c]);
-      ZR[(size_t)g * N + n + c] = as_u16((f16)zr[c]);
+      float q[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) q[j] = code_of<decltype(div)::value>(r[j].at(c), qc[c]);
+      word[c] = pack_codes(q);
+    }
+    uint32_t* dst = QW + (size_t)(g * octs + o) * N + n;
+    if constexpr (VEC) {
+      *reinterpret_cast<uint4*>(dst) = make_uint4(word[0], word[1], word[2], word[3]);
+    } else {
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        if (c < left) dst[c * kStep] = word[c];
+    }
+  };
+  auto all_codes = [&](auto div) {
+    if constexpr (OPW > 0) {
+#pragma unroll
+      for (int i = 0; i < OPW; ++i)
+        if (o0 + i < o1) codes(div, keep[i], o0 + i);
+    } else {
+      for (int o = o0; o < o1; ++o) {
+        load8(keep[0], o);
+        codes(div, keep[0], o);
+      }
+    }
+  };
+  if (__all(fast)) all_codes(std::false_type{});
+  else all_codes(std::true_type{});
+  if (part == 0) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      if (c < left) {
+        SC[(size_t)g * N + n + c * kStep] = as_u16((f16)qc[c].s);
+        ZR[(size_t)g * N + n + c * kStep] = as_u16((f16)qc[c].z);
+      }
     }
   }
 }
@@ -461,6 +523,28 @@ __global__ __launch_bounds__(256) void zeros_check_kernel(const f16* __restrict_
   if (bad) *flag = 1;
 }
 
+template <class IN, bool VEC>
+hipError_t quantize_tile_launch(const typename IN::T* w, uint32_t* q, uint16_t* s, uint16_t* z,
+                                int K, int N, int G, int32_t* flag, hipStream_t st) {
+  // Waves per group and octets per wave, so that a wave keeps about four
+  // octets (32 rows) in registers whatever G: one wave per group up to G = 32,
+  // two at 64, four beyond; more than 8 (fp16) / 4 (fp32) octets a wave are
+  // read twice.
+  const int octs = G / 8, per = (octs + 3) / 4;
+  constexpr int kMaxKeep = sizeof(typename IN::T) == 2 ? 8 : 4;
+  const int gpb = octs <= 4 ? 4 : octs <= 8 ? 2 : 1;   // groups per workgroup
+  auto k = octs <= 1   ? quantize_tile_kernel<IN, 1, 1, VEC>
+           : octs <= 2 ? quantize_tile_kernel<IN, 2, 1, VEC>
+           : octs <= 4 ? quantize_tile_kernel<IN, 4, 1, VEC>
+           : octs <= 8 ? quantize_tile_kernel<IN, 4, 2, VEC>
+           : per <= 4  ? quantize_tile_kernel<IN, 4, 4, VEC>
+           : per <= kMaxKeep ? quantize_tile_kernel<IN, kMaxKeep, 4, VEC>
+                             : quantize_tile_kernel<IN, 0, 4, VEC>;
+  const unsigned blocks = (unsigned)((K / G + gpb - 1) / gpb) * (unsigned)((N + 255) / 256);
+  hipLaunchKernelGGL(k, dim3(blocks), dim3(256), 0, st, w, q, s, z, K, N, G, flag);
+  return hipGetLastError();
+}
+
 template <class IN>
 hipError_t quantize_launch(const void* W, int32_t* qw, void* sc, void* zr, int K, int N, int G,
                            int32_t* flag, hipStream_t st) {
@@ -478,24 +562,8 @@ hipError_t quantize_launch(const void* W, int32_t* qw, void* sc, void* zr, int K
   const uintptr_t wa = 4 * sizeof(T);
   const bool vec = (N % 4 == 0) && ((reinterpret_cast<uintptr_t>(W) & (wa - 1)) == 0) &&
                    ((reinterpret_cast<uintptr_t>(qw) & 15) == 0);
-  if (vec) {
-    // octets per wave: kept in registers up to 8 (fp16) / 4 (fp32), beyond
-    // that read twice
-    const int per = (G / 8 + 3) / 4;
-    constexpr int kMaxKeep = sizeof(T) == 2 ? 8 : 4;
-    auto k = per <= 1 ? quantize_tile_kernel<IN, 1>
-             : per <= 2 ? quantize_tile_kernel<IN, 2>
-             : per <= 4 ? quantize_tile_kernel<IN, 4>
-             : per <= kMaxKeep ? quantize_tile_kernel<IN, kMaxKeep>
-                              : quantize_tile_kernel<IN, 0>;
-    dim3 grid(K / G, (N + 255) / 256);
-    hipLaunchKernelGGL(k, grid, dim3(256), 0, st, w, q, s, z, K, N, G, flag);
-  } else {
-    dim3 grid(K / G, (N + 255) / 256);
-    hipLaunchKernelGGL((quantize_kernel<IN, 1>), grid, dim3(256), 0, st, w, q, s, z, K, N, G,
-                       flag);
-  }
-  return hipGetLastError();
+  return vec ? quantize_tile_launch<IN, true>(w, q, s, z, K, N, G, flag, st)
+             : quantize_tile_launch<IN, false>(w, q, s, z, K, N, G, flag, st);
 }
 
 }  // namespace
