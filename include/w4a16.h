@@ -235,6 +235,17 @@ int w4a16_quantize_pack_f32(const void* W, int32_t* qweight, void* scales, void*
                             void* stream);
 
 /*
+ * Quantise W given transposed: W[n * ldw + k], the layout of an nn.Linear
+ * weight [N, K] (fp32 if w_is_f32, else fp16), to the same results as
+ * w4a16_quantize_pack_* on its [K, N] copy, without making that copy.  Needs
+ * N >= 2, ldw >= K, 16-byte aligned rows and group_size 32, 64, 128, 256 or
+ * 512; W4A16_ERR_BAD_PLAN otherwise (nothing is launched).
+ */
+int w4a16_quantize_pack_nk(const void* W, int32_t w_is_f32, int64_t ldw, int32_t* qweight,
+                           void* scales, void* zeros, int64_t K, int64_t N, int64_t group_size,
+                           int32_t* flag, void* stream);
+
+/*
  * pack_int4 (w4a16-kernel/src/w4a16/quant.py:45-70): int32 codes [K, N] ->
  * int32 [K/8, N].  `flag` (caller zero-filled) is set to 1 if a code lies
  * outside [0, 15] (the reference asserts, quant.py:62-63).

@@ -148,6 +148,30 @@ def test_quantize_ties_and_scales_every_group_split(G, dtype, N):
     _assert_quant_equal(torch.from_numpy(W).to(dtype), G, f"ties G={G} N={N}")
 
 
+@pytest.mark.parametrize("G", [32, 64, 96, 128, 256, 512])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32, torch.bfloat16])
+def test_quantize_transposed_weight(G, dtype):
+    """A W whose columns are contiguous (an nn.Linear weight's transpose) is read
+    in place: partial 512-k chunks and column tiles, rows longer than K, ties,
+    scales outside the corrected-reciprocal range, zero minima of either sign,
+    and the layouts that are copied first (G = 96, rows off 16 bytes, N = 1)."""
+    log(f"quantize transposed G={G} {dtype}")
+    rng = np.random.default_rng(G)
+    for K, N, pad, off in ((3 * G, 2, 0, 0), (5 * G, 67, 8, 0), (7 * G, 130, 0, 0), (2 * G, 64, 0, 1),
+                           (2 * G, 33, 4, 0), (2 * G, 1, 8, 0)):
+        W = rng.integers(-16, 17, (N, K + pad)).astype(np.float32) * 0.5
+        W *= np.exp2(rng.integers(-4, 1, (N, 1)))
+        W[::3] = np.abs(W[::3])
+        W[::3] = np.where(W[::3] == 0, np.where(rng.random(W[::3].shape) < 0.5, -0.0, 0.0), W[::3])
+        W[1::5] += rng.standard_normal(W[1::5].shape) * 0.01
+        if dtype == torch.float32:
+            W[2::7] *= np.float32(2.0 ** -110)
+        flat = torch.zeros(N * (K + pad) + off, dtype=dtype, device=DEV)
+        flat[off:] = torch.from_numpy(W).to(dtype).to(DEV).reshape(-1)
+        view = flat[off:].view(N, K + pad)[:, :K].t()
+        _assert_quant_equal(view.float() if dtype == torch.bfloat16 else view, G, f"transposed {K}x{N}")
+
+
 def test_quantize_fp32_tiny_and_denormal_ranges():
     log("quantize fp32 tiny ranges")
     K, N, G = 64, 8, 32

@@ -1326,6 +1326,19 @@ int w4a16_quantize_pack_f32(const void* W, int32_t* qweight, void* scales, void*
   return quantize_common(W, true, qweight, scales, zeros, K, N, group_size, flag, stream);
 }
 
+int w4a16_quantize_pack_nk(const void* W, int32_t w_is_f32, int64_t ldw, int32_t* qweight,
+                           void* scales, void* zeros, int64_t K, int64_t N, int64_t group_size,
+                           int32_t* flag, void* stream) {
+  if (int st = check_gemm_shape(0, N, K, group_size)) return st;
+  if (K == 0 || N == 0) return W4A16_OK;
+  if (!W || !qweight || !scales || !zeros || !flag) return W4A16_ERR_NULL_POINTER;
+  if (!quantize_nk_applicable(W, w_is_f32 != 0, ldw, (int)K, (int)N, (int)group_size))
+    return W4A16_ERR_BAD_PLAN;
+  return to_status(launch_quantize_pack_nk(W, w_is_f32 != 0, ldw, qweight, scales, zeros, (int)K,
+                                           (int)N, (int)group_size, flag,
+                                           static_cast<hipStream_t>(stream)));
+}
+
 int w4a16_pack_int4(const int32_t* q, int32_t* qweight, int64_t K, int64_t N, int32_t* flag,
                     void* stream) {
   if (int st = check_gemm_shape(0, N, K, 8)) return st;

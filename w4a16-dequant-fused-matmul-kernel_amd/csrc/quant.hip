@@ -402,6 +402,207 @@ __global__ __launch_bounds__(256) void quantize_tile_kernel(const typename IN::T
   }
 }
 
+// v from another lane of the same group of L consecutive lanes, step D of a
+// butterfly (D = 1, 2, 4, 8 by DPP: within quads, mirrored halves and rows of
+// 16 lanes; 16 and 32 through the LDS crossbar).
+template <int D>
+__device__ __forceinline__ uint32_t lane_swap(uint32_t v) {
+  if constexpr (D >= 16) {
+    return (uint32_t)__shfl_xor((int)v, D);
+  } else {
+    constexpr int ctrl = D == 1 ? 0xB1 : D == 2 ? 0x4E : D == 4 ? 0x141 : 0x140;
+    return (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, ctrl, 0xF, 0xF, false);
+  }
+}
+
+// Eight consecutive k of one column (a packed word's worth): loads, minimum and
+// maximum over L lanes (IEEE minimum / maximum, as MinMax4).
+template <class IN>
+struct Oct;
+template <>
+struct Oct<InF16> {
+  uint4 v;
+  __device__ __forceinline__ void load(const uint16_t* p) { v = *reinterpret_cast<const uint4*>(p); }
+  // keeps the compiler from carrying converted copies of the weights (twice
+  // their registers) from one pass
+  // over them to the next
+  __device__ __forceinline__ void hide() { asm("" : "+v"(v.x), "+v"(v.y), "+v"(v.z), "+v"(v.w)); }
+  __device__ __forceinline__ f16 at(int j) const {
+    const f16x2 h = as_h2(j < 2 ? v.x : j < 4 ? v.y : j < 6 ? v.z : v.w);
+    return j & 1 ? h.y : h.x;
+  }
+  template <int L>
+  __device__ __forceinline__ void min_max(float& mn, float& mx) const {
+    const f16x2 a = as_h2(v.x), b = as_h2(v.y), c = as_h2(v.z), d = as_h2(v.w);
+    f16x2 lo = __builtin_elementwise_minimum(
+        __builtin_elementwise_minimum(a, b), __builtin_elementwise_minimum(c, d));
+    f16x2 hi = __builtin_elementwise_maximum(
+        __builtin_elementwise_maximum(a, b), __builtin_elementwise_maximum(c, d));
+    auto fold = [&](auto step) {
+      constexpr int D = decltype(step)::value;
+      if constexpr (D < L) {
+        lo = __builtin_elementwise_minimum(lo, as_h2(lane_swap<D>(as_u32(lo))));
+        hi = __builtin_elementwise_maximum(hi, as_h2(lane_swap<D>(as_u32(hi))));
+      }
+    };
+    fold(std::integral_constant<int, 1>{});
+    fold(std::integral_constant<int, 2>{});
+    fold(std::integral_constant<int, 4>{});
+    fold(std::integral_constant<int, 8>{});
+    fold(std::integral_constant<int, 16>{});
+    fold(std::integral_constant<int, 32>{});
+    mn = __builtin_elementwise_minimum((float)lo.x, (float)lo.y);
+    mx = __builtin_elementwise_maximum((float)hi.x, (float)hi.y);
+  }
+};
+template <>
+struct Oct<InF32> {
+  float4 a, b;
+  __device__ __forceinline__ void load(const float* p) {
+    a = reinterpret_cast<const float4*>(p)[0];
+    b = reinterpret_cast<const float4*>(p)[1];
+  }
+  __device__ __forceinline__ void hide() {}
+  __device__ __forceinline__ float at(int j) const {
+    const float4 f = j < 4 ? a : b;
+    return (j & 3) == 0 ? f.x : (j & 3) == 1 ? f.y : (j & 3) == 2 ? f.z : f.w;
+  }
+  template <int L>
+  __device__ __forceinline__ void min_max(float& mn, float& mx) const {
+    mn = mx = at(0);
+#pragma unroll
+    for (int j = 1; j < 8; ++j) {
+      mn = __builtin_elementwise_minimum(mn, at(j));
+      mx = __builtin_elementwise_maximum(mx, at(j));
+    }
+    auto fold = [&](auto step) {
+      constexpr int D = decltype(step)::value;
+      if constexpr (D < L) {
+        mn = __builtin_elementwise_minimum(
+            mn, __builtin_bit_cast(float, lane_swap<D>(__builtin_bit_cast(uint32_t, mn))));
+        mx = __builtin_elementwise_maximum(
+            mx, __builtin_bit_cast(float, lane_swap<D>(__builtin_bit_cast(uint32_t, mx))));
+      }
+    };
+    fold(std::integral_constant<int, 1>{});
+    fold(std::integral_constant<int, 2>{});
+    fold(std::integral_constant<int, 4>{});
+    fold(std::integral_constant<int, 8>{});
+    fold(std::integral_constant<int, 16>{});
+    fold(std::integral_constant<int, 32>{});
+  }
+};
+
+// Quantise from the transposed weight: column n's K weights lie in a row of
+// `ldw` elements (an nn.Linear weight [N, K]), so no transposed copy of W is
+// made first.  G = 8 L, L a power of two from 4 to 64.  A workgroup of 4 waves
+// takes 32 columns x 512 k: a wave reads one column's 512 k as one contiguous
+// kilobyte (fp16), lane l holding the 8 k of one packed word; the L lanes of a
+// group find its minimum and maximum by a butterfly, each of them finishes one
+// column's (or several columns') scale and zero-point, and the words are turned
+// round through LDS (rows padded by a word, no bank conflicts) so that they
+// leave as runs of 32 adjacent words.  A zero minimum takes the sign of the
+// first or last zero in k order (min_step), found from the wave's ballots.
+// Bound by memory.  Measured on MI355X, us, kernel alone: K = 4096, N = 11008 /
+// 14336, G = 128 29.9 / 35.2 (4.2 TB/s), fp32 N = 14336 44.8 (6.0 TB/s), K =
+// 8192, N = 28672 116.9; before, a transposing copy (292 at N = 11008) and the
+// row-major quantiser.  16 columns a wave (runs of 64 words, 133 registers, three
+// waves per SIMD) took 33.7 / 38.6.
+constexpr int kNkCols = 8;   // columns per wave
+template <class IN, int L>
+__global__ __launch_bounds__(256) void quantize_nk_kernel(const typename IN::T* __restrict__ W,
+                                                          int64_t ldw, uint32_t* __restrict__ QW,
+                                                          uint16_t* __restrict__ SC,
+                                                          uint16_t* __restrict__ ZR, int K, int N,
+                                                          int32_t* __restrict__ flag) {
+  static_assert(L >= 4 && L <= 64 && (L & (L - 1)) == 0, "a group is L lanes of a wave");
+  constexpr int R = kNkCols, kCols = 4 * R;
+  constexpr int kGrp = 64 / L;                     // groups in a wave's 512 k
+  constexpr int kOwn = L >= R ? 1 : R / L;         // columns a lane finishes
+  __shared__ uint32_t words[64][kCols + 1];
+  __shared__ float4 stat[4][R][kGrp];              // s, r, z, fast_scale
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int nkc = (K + 511) / 512;
+  const int kc = (int)(blockIdx.x % (unsigned)nkc);
+  const int n0 = (int)(blockIdx.x / (unsigned)nkc) * kCols;
+  const int k = kc * 512 + 8 * lane;
+  const bool kv = k < K;                           // whole groups: K % G == 0
+  const int sub = lane % L, grp = lane / L;
+
+  // Lanes past K and columns past N load in-range weights whose results go
+  // nowhere: under a branch each load would be waited for before the next.
+  Oct<IN> v[R];
+#pragma unroll
+  for (int i = 0; i < R; ++i)
+    v[i].load(W + (size_t)min(N - 1, n0 + wave * R + i) * ldw + (kv ? k : 0));
+  float omn[kOwn] = {}, omx[kOwn] = {};
+  bool bad = false;
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    float mn, mx;
+    v[i].template min_max<L>(mn, mx);
+    bad |= !finite(mn) || !finite(mx);
+    if (__any(mn == 0.0f)) {
+      const bool last = n0 + wave * R + i < 32 * (N / 32);
+      float z = __builtin_inff();
+      v[i].hide();
+#pragma unroll
+      for (int j = 0; j < 8; ++j) z = min_step((float)v[i].at(j), z, last);
+      const uint64_t has = __ballot(z == 0.0f);
+      const uint64_t neg = __ballot(z == 0.0f && __builtin_signbit(z));
+      const uint64_t mine = (has >> (grp * L)) & (L == 64 ? ~0ull : (1ull << (L % 64)) - 1ull);
+      if (mn == 0.0f) {
+        const int at = grp * L + (last ? 63 - __builtin_clzll(mine) : __builtin_ctzll(mine));
+        mn = (neg >> at) & 1ull ? -0.0f : 0.0f;
+      }
+    }
+    if (sub == i % L) {
+      omn[i / L] = mn;
+      omx[i / L] = mx;
+    }
+  }
+  if (bad) *flag = 1;
+#pragma unroll
+  for (int o = 0; o < kOwn; ++o) {
+    const int i = o * L + sub;
+    if (i < R) {
+      const QCol c = make_qcol(omn[o], omx[o]);
+      stat[wave][i][grp] = make_float4(c.s, c.r, c.z, fast_scale(c.s) ? 1.0f : 0.0f);
+      const int n = n0 + wave * R + i;
+      if (kv && n < N) {
+        const size_t at = (size_t)(kc * kGrp + grp) * N + n;
+        SC[at] = as_u16((f16)c.s);
+        ZR[at] = as_u16((f16)c.z);
+      }
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    v[i].hide();
+    const float4 st = stat[wave][i][grp];
+    const QCol c{st.x, st.y, st.z};
+    float q[8];
+    if (__all(st.w != 0.0f)) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) q[j] = code_of<false>(v[i].at(j), c);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) q[j] = code_of<true>(v[i].at(j), c);
+    }
+    words[lane][wave * R + i] = pack_codes(q);
+  }
+  __syncthreads();
+  constexpr int kRows = 256 / kCols;               // packed rows written at once
+  const int wc = threadIdx.x % kCols, wr = threadIdx.x / kCols;
+#pragma unroll
+  for (int o = 0; o < 64; o += kRows) {
+    const int row = kc * 64 + o + wr;
+    if (row < K / 8 && n0 + wc < N) QW[(size_t)row * N + n0 + wc] = words[o + wr][wc];
+  }
+}
+
 // Any G dividing K (G % 8 != 0 lets a packed word straddle groups): one thread
 // per packed word; each row's group statistics are recomputed from the group's
 // G values, and the thread that owns a group's first row writes its scale/zero.
@@ -566,12 +767,42 @@ hipError_t quantize_launch(const void* W, int32_t* qw, void* sc, void* zr, int K
              : quantize_tile_launch<IN, false>(w, q, s, z, K, N, G, flag, st);
 }
 
+template <class IN>
+hipError_t quantize_nk_launch(const void* W, int64_t ldw, int32_t* qw, void* sc, void* zr, int K,
+                              int N, int G, int32_t* flag, hipStream_t st) {
+  auto k = G == 32    ? quantize_nk_kernel<IN, 4>
+           : G == 64  ? quantize_nk_kernel<IN, 8>
+           : G == 128 ? quantize_nk_kernel<IN, 16>
+           : G == 256 ? quantize_nk_kernel<IN, 32>
+                      : quantize_nk_kernel<IN, 64>;
+  const unsigned blocks = (unsigned)((K + 511) / 512) * (unsigned)((N + 4 * kNkCols - 1) / (4 * kNkCols));
+  hipLaunchKernelGGL(k, dim3(blocks), dim3(256), 0, st, static_cast<const typename IN::T*>(W), ldw,
+                     reinterpret_cast<uint32_t*>(qw), static_cast<uint16_t*>(sc),
+                     static_cast<uint16_t*>(zr), K, N, flag);
+  return hipGetLastError();
+}
+
 }  // namespace
 
 hipError_t launch_quantize_pack(const void* W, bool w_is_f32, int32_t* qw, void* sc, void* zr,
                                 int K, int N, int G, int32_t* flag, hipStream_t st) {
   return w_is_f32 ? quantize_launch<InF32>(W, qw, sc, zr, K, N, G, flag, st)
                   : quantize_launch<InF16>(W, qw, sc, zr, K, N, G, flag, st);
+}
+
+bool quantize_nk_applicable(const void* W, bool w_is_f32, int64_t ldw, int K, int N, int G) {
+  // rows of whole 16-byte loads; N == 1 has its own zero rule (inner_zero_min)
+  const int64_t elems = w_is_f32 ? 4 : 8;
+  return N >= 2 && ldw >= K && ldw % elems == 0 && K % 8 == 0 &&
+         (reinterpret_cast<uintptr_t>(W) & 15) == 0 &&
+         (G == 32 || G == 64 || G == 128 || G == 256 || G == 512) && K % G == 0;
+}
+
+hipError_t launch_quantize_pack_nk(const void* W, bool w_is_f32, int64_t ldw, int32_t* qw,
+                                   void* sc, void* zr, int K, int N, int G, int32_t* flag,
+                                   hipStream_t st) {
+  return w_is_f32 ? quantize_nk_launch<InF32>(W, ldw, qw, sc, zr, K, N, G, flag, st)
+                  : quantize_nk_launch<InF16>(W, ldw, qw, sc, zr, K, N, G, flag, st);
 }
 
 hipError_t launch_pack(const int32_t* q, int32_t* qw, int K, int N, int32_t* flag,

@@ -130,6 +130,12 @@ hipError_t launch_simt(const GemmArgs& a, hipStream_t st);
 // Quantisation / packing kernels.
 hipError_t launch_quantize_pack(const void* W, bool w_is_f32, int32_t* qw, void* sc, void* zr,
                                 int K, int N, int G, int32_t* flag, hipStream_t st);
+// The same from W transposed, [N, K] in rows of ldw elements; only where
+// quantize_nk_applicable.
+bool quantize_nk_applicable(const void* W, bool w_is_f32, int64_t ldw, int K, int N, int G);
+hipError_t launch_quantize_pack_nk(const void* W, bool w_is_f32, int64_t ldw, int32_t* qw,
+                                   void* sc, void* zr, int K, int N, int G, int32_t* flag,
+                                   hipStream_t st);
 hipError_t launch_pack(const int32_t* q, int32_t* qw, int K, int N, int32_t* flag, hipStream_t st);
 hipError_t launch_unpack(const int32_t* qw, int32_t* q, int K, int N, hipStream_t st);
 hipError_t launch_dequant(const int32_t* qw, const void* sc, const void* zr, void* w, int K,

@@ -43,6 +43,9 @@ STATUS = {
 }
 
 
+ERR_BAD_PLAN = -5
+
+
 class Plan(ctypes.Structure):
     """Mirror of ``struct w4a16_plan``."""
 
@@ -97,6 +100,7 @@ SIGNATURES = {
     ),
     "w4a16_quantize_pack_f16": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp, _vp]),
     "w4a16_quantize_pack_f32": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp, _vp]),
+    "w4a16_quantize_pack_nk": (_int, [_vp, _i32, _i64, _vp, _vp, _vp, _i64, _i64, _i64, _vp, _vp]),
     "w4a16_pack_int4": (_int, [_vp, _vp, _i64, _i64, _vp, _vp]),
     "w4a16_unpack_int4": (_int, [_vp, _vp, _i64, _i64, _vp]),
     "w4a16_dequantize_f16": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp]),

@@ -82,12 +82,22 @@ class W4A16Linear(nn.Module):
         same device; its bias, if any, converted to fp16."""
         out_features, in_features = linear.weight.shape
         has_bias = linear.bias is not None
-        layer = cls(in_features, out_features, group_size=group_size, bias=has_bias,
-                    device=linear.weight.device)
-        # [out, in] -> the [K, N] layout quantize_weight expects
-        layer.quantize_from_dense(linear.weight.detach().t().contiguous())
+        # [out, in] seen as the [K, N] quantize_weight expects; its transposed
+        # rows are read in place
+        W = linear.weight.detach().t()
+        if cls is not W4A16Linear:
+            layer = cls(in_features, out_features, group_size=group_size, bias=has_bias,
+                        device=linear.weight.device)
+            layer.quantize_from_dense(W.contiguous())
+            if has_bias:
+                layer.bias.copy_(linear.bias.detach().to(torch.float16))
+            return layer
+        # a fresh layer takes the quantiser's tensors as its buffers: nothing is
+        # zeroed first or copied afterwards
+        layer = cls(in_features, out_features, group_size=group_size, bias=has_bias, device="meta")
+        layer.qweight, layer.scales, layer.zeros = quantize_weight(W, group_size)
         if has_bias:
-            layer.bias.copy_(linear.bias.detach().to(torch.float16))
+            layer.bias = linear.bias.detach().to(W.device, torch.float16, copy=True).contiguous()
         return layer
 
     def quantize_from_dense(self, W: Tensor) -> None:

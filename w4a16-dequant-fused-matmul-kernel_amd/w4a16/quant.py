@@ -79,6 +79,24 @@ def unpack_int4(qweight: Tensor, K: int | None = None) -> Tensor:
     return out.to(home)
 
 
+def _quantize_pack(W: Tensor, qweight: Tensor, scales: Tensor, zeros: Tensor, G: int,
+                   flag: Tensor) -> int:
+    """Launch the quantiser on a device W of fp16 or fp32; the status.  A W whose
+    columns are the contiguous direction (a transposed nn.Linear weight) is read
+    as it lies where the kernel for that layout takes it, else copied first."""
+    K, N = W.shape
+    f32 = W.dtype == torch.float32
+    rest = (qweight.data_ptr(), scales.data_ptr(), zeros.data_ptr(), K, N, G, flag.data_ptr(),
+            rt.stream_ptr(W.device))
+    if W.stride(0) == 1 and W.stride(1) >= K and not W.is_contiguous():
+        code = rt.lib().w4a16_quantize_pack_nk(W.data_ptr(), int(f32), W.stride(1), *rest)
+        if code != _lib.ERR_BAD_PLAN:
+            return code
+    W = W.contiguous()
+    fn = rt.lib().w4a16_quantize_pack_f32 if f32 else rt.lib().w4a16_quantize_pack_f16
+    return fn(W.data_ptr(), *rest)
+
+
 def quantize_weight(W: Tensor, group_size: int = 128) -> tuple[Tensor, Tensor, Tensor]:
     """Group-wise asymmetric 4-bit quantisation of ``W`` [K, N] along K (quant.py:101-144).
 
@@ -100,16 +118,12 @@ def quantize_weight(W: Tensor, group_size: int = 128) -> tuple[Tensor, Tensor, T
     with rt.on_device(dev):
         if Wd.dtype not in (torch.float16, torch.float32):
             Wd = Wd.to(torch.float32)
-        Wd = Wd.contiguous()
-        fn = (rt.lib().w4a16_quantize_pack_f32 if Wd.dtype == torch.float32
-              else rt.lib().w4a16_quantize_pack_f16)
         qweight = torch.empty((K // _NIBBLES_PER_INT32, N), dtype=torch.int32, device=dev)
         scales = torch.empty((K // G, N), dtype=torch.float16, device=dev)
         zeros = torch.empty((K // G, N), dtype=torch.float16, device=dev)
         if Wd.numel():
             flag = _flag(dev)
-            _lib.check(fn(Wd.data_ptr(), qweight.data_ptr(), scales.data_ptr(), zeros.data_ptr(),
-                          K, N, G, flag.data_ptr(), rt.stream_ptr(dev)), "w4a16_quantize_pack")
+            _lib.check(_quantize_pack(Wd, qweight, scales, zeros, G, flag), "w4a16_quantize_pack")
             if int(flag.item()) != 0:
                 raise AssertionError(
                     "uint4 values must be in [0,15]: W holds a non-finite value")
