@@ -300,6 +300,30 @@ def test_dequant_bit_exact(K, N, G):
     assert np.array_equal(np_(out).view(np.uint16), ref.view(np.uint16))
 
 
+@pytest.mark.parametrize("N,off", [(8, 0), (2056, 0), (4, 0), (1028, 0), (2048, 4), (2048, 2), (1027, 0)])
+@pytest.mark.parametrize("G", [8, 40, 128])
+def test_dequant_columns_per_lane(N, off, G):
+    """8, 4 or 1 columns a lane by N and the alignment of scales and zeros (off =
+    their offset in elements), partial column blocks, and zero-points and scales
+    of every magnitude, infinities and NaN included, to the oracle's bits."""
+    from w4a16 import dequantize_weight
+
+    log(f"dequant columns N={N} off={off} G={G}")
+    K = 3 * G
+    rng = np.random.default_rng(N + off + G)
+    qw = torch.from_numpy(rng.integers(-2**31, 2**31, (K // 8, N)).astype(np.int32))
+    buf = torch.from_numpy(rng.integers(0, 2**16, 2 * 3 * N + 2 * off).astype(np.uint16).view(np.float16))
+    s, z = buf[off:off + 3 * N].view(3, N), buf[2 * off + 3 * N:].view(3, N)
+    dev = buf.to(DEV)
+    out = dequantize_weight(qw.to(DEV), dev[off:off + 3 * N].view(3, N),
+                            dev[2 * off + 3 * N:].view(3, N), G)
+    with np.errstate(all="ignore"):
+        ref = O.dequantize_weight(qw.numpy(), s.numpy(), z.numpy(), G)
+    got, nan = np_(out), np.isnan(ref)
+    assert np.array_equal(np.isnan(got), nan)
+    assert np.array_equal(got.view(np.uint16)[~nan], ref.view(np.uint16)[~nan])
+
+
 def test_quant_dequant_roundtrip_error():
     """Reference test_quant.py:71-90 on the device: mean relative error < 0.15."""
     from w4a16 import dequantize_weight, quantize_weight

@@ -710,6 +710,59 @@ __global__ __launch_bounds__(256) void dequant_kernel(const uint32_t* __restrict
   }
 }
 
+// dequantize_weight, C = 8 or 4 adjacent columns of one packed row per lane (G %
+// 8 == 0: one group): 16-byte weight loads, and rows stored 2 C bytes per lane,
+// so that a wave writes 1024 or 512 contiguous bytes of a row.  Two columns'
+// codes of one row make a packed pair: byte b of both words (v_perm_b32) holds
+// rows 2b and 2b + 1 as nibbles, which the magic words turn into the fp16 pairs
+// 1024 + q and 64 + q; the magic is subtracted first (exact), then (q - z) * s is
+// rounded as dequant_kernel rounds it.  Bound by memory, mostly by
+// the stores, which are non-temporal (W is written once, and need not pass
+// through L2).  Measured on MI355X with cold operands, us, one column a lane ->
+// this with plain stores -> non-temporal: K = 4096, N = 11008 / 14336 42.7 / 54.0
+// -> 25.4 / 28.8 -> 17.0 / 23.7 (6.3-6.7 TB/s); K = 8192, N = 28672 213 -> 104 ->
+// 91.6; four columns, N = 11004 42.5 -> 27.6 -> 25.2.
+template <int C>
+__global__ __launch_bounds__(256) void dequant_vec_kernel(const uint32_t* __restrict__ QW,
+                                                          const uint16_t* __restrict__ SC,
+                                                          const uint16_t* __restrict__ ZR,
+                                                          uint16_t* __restrict__ Wd, int N,
+                                                          int octs) {
+  static_assert(C == 4 || C == 8, "one or two 16-byte weight loads");
+  typedef uint32_t Vec __attribute__((ext_vector_type(C / 2)));   // C halves
+  const int nblk = (N + 256 * C - 1) / (256 * C);
+  const int i = (int)(blockIdx.x / (unsigned)nblk);               // packed row
+  const int n = ((int)(blockIdx.x % (unsigned)nblk) * 256 + (int)threadIdx.x) * C;
+  if (n >= N) return;
+  const size_t at = (size_t)(i / octs) * N + n;
+  uint32_t w[C];
+#pragma unroll
+  for (int c = 0; c < C; c += 4) {
+    const uint4 v = *reinterpret_cast<const uint4*>(QW + (size_t)i * N + n + c);
+    w[c] = v.x, w[c + 1] = v.y, w[c + 2] = v.z, w[c + 3] = v.w;
+  }
+  const Vec s = *reinterpret_cast<const Vec*>(SC + at);
+  const Vec z = *reinterpret_cast<const Vec*>(ZR + at);
+  const MagicRegs mg = make_magic();
+  uint16_t* dst = Wd + (size_t)i * 8 * N + n;
+#pragma unroll
+  for (int b = 0; b < 4; ++b) {
+    Vec even, odd;
+#pragma unroll
+    for (int c = 0; c < C / 2; ++c) {
+      // byte b of column 2c into byte 0, of column 2c + 1 into byte 2
+      const uint32_t t = __builtin_amdgcn_perm(w[2 * c + 1], w[2 * c],
+                                               0x0C040C00u + 0x00010001u * (uint32_t)b);
+      const f16x2 lo = as_h2(and_or(t, 0x000F000Fu, mg.m1024)) - as_h2(mg.m1024);
+      const f16x2 hi = as_h2(and_or(t, 0x00F000F0u, mg.m64)) - as_h2(mg.m64);
+      even[c] = as_u32((lo - as_h2(z[c])) * as_h2(s[c]));
+      odd[c] = as_u32((hi - as_h2(z[c])) * as_h2(s[c]));
+    }
+    __builtin_nontemporal_store(even, reinterpret_cast<Vec*>(dst + (size_t)(2 * b) * N));
+    __builtin_nontemporal_store(odd, reinterpret_cast<Vec*>(dst + (size_t)(2 * b + 1) * N));
+  }
+}
+
 // Zero-points outside the integer-zero kernels' domain (w4a16_device.h): any
 // zero that is not an integer in [-1024, 1024] (NaN and infinities included)
 // sets *flag.  Grid-stride over the n halves; every offending lane stores 1.
@@ -829,6 +882,24 @@ hipError_t launch_zeros_check(const void* zr, int64_t n, int32_t* flag, hipStrea
 
 hipError_t launch_dequant(const int32_t* qw, const void* sc, const void* zr, void* w, int K,
                           int N, int G, hipStream_t st) {
+  // 8 columns a lane where rows and pointers allow its 16-byte accesses, 4 where
+  // they allow 8-byte ones; else (and where a packed row holds two groups) one
+  auto ok = [&](int c) {
+    const uintptr_t m = 2 * (uintptr_t)c - 1;
+    return N % c == 0 && G % 8 == 0 &&
+           (((reinterpret_cast<uintptr_t>(sc) | reinterpret_cast<uintptr_t>(zr) |
+              reinterpret_cast<uintptr_t>(w)) & m) |
+            (reinterpret_cast<uintptr_t>(qw) & 15)) == 0;
+  };
+  const int c = ok(8) ? 8 : ok(4) ? 4 : 1;
+  const unsigned blocks = (unsigned)(K / 8) * (unsigned)((N + 256 * c - 1) / (256 * c));
+  if (c > 1) {
+    hipLaunchKernelGGL((c == 8 ? dequant_vec_kernel<8> : dequant_vec_kernel<4>), dim3(blocks),
+                       dim3(256), 0, st, reinterpret_cast<const uint32_t*>(qw),
+                       static_cast<const uint16_t*>(sc), static_cast<const uint16_t*>(zr),
+                       static_cast<uint16_t*>(w), N, G / 8);
+    return hipGetLastError();
+  }
   dim3 grid(K / 8, (N + 255) / 256);
   hipLaunchKernelGGL(dequant_kernel, grid, dim3(256), 0, st,
                      reinterpret_cast<const uint32_t*>(qw), static_cast<const f16*>(sc),
