@@ -284,13 +284,13 @@ def _prepare(case, copies_for_cold: bool):
 
 def bench_case(case, steps: int, warmup: int, graph: bool = False, cold: bool = True) -> dict:
     from w4a16 import w4a16_matmul
-    from w4a16.hip_kernel import plan_for
+    from w4a16 import _lib
 
     X, W, Xd, layers, y, ncopy, per_copy = _prepare(case, cold)
     fns = [(lambda l=l: w4a16_matmul(Xd, l[0], l[1], l[2], case.G, out=y)) for l in layers]
     t = _time_calls(fns, steps, warmup, graph)
     ms = t["ms"]
-    p = plan_for(case.M, case.N, case.K, case.G).as_dict()
+    p = _lib.auto_plan(case.M, case.N, case.K, case.G).as_dict()
     us = ms * 1e3
     gbs = case.bytes() / (ms * 1e-3) / 1e9
     tflops = case.flops() / (ms * 1e-3) / 1e12

@@ -65,7 +65,7 @@ enum w4a16_kernel {
 /* w4a16_plan.flags */
 #define W4A16_PLAN_ANY_ZEROS 1 /* zeros may be any fp16 value (see above)     */
 
-/* The launch a GEMM call will make.  Filled by w4a16_gemm_plan(). */
+/* The launch a planned GEMM call will make.  Filled by w4a16_gemm_plan(). */
 typedef struct w4a16_plan {
   int32_t kernel;          /* enum w4a16_kernel (never AUTO once planned)       */
   int32_t split_k;         /* GEMV, MFMA cfg 7/11-14: k-splits (1 = none)       */
@@ -130,7 +130,22 @@ int w4a16_gemm_plan(int64_t M, int64_t N, int64_t K, int64_t group_size, int32_t
  */
 int w4a16_zeros_check_f16(const void* zeros, int64_t count, int32_t* flag, void* stream);
 
-/* Workspace bytes the automatic plan for this shape needs (0 = none). */
+/*
+ * What an automatic call (w4a16_gemm_f16, w4a16_linear_f16, w4a16_gemm_f16_auto,
+ * and w4a16_gemm_f16_strided without a plan) runs for a shape, given aligned
+ * operands and the workspace below.  (w4a16_gemm_f16_noalloc runs
+ * w4a16_gemm_plan's.)  Prefill shapes (M > 32), and widths
+ * or alignments the planned kernels do not take, run the one-wave-per-SIMD
+ * prefill kernel, reported as MFMA tile_cfg 16 .. 20 (256 x 256, 128 x 256, and,
+ * with k-slices inside the workgroup, 128 x 128, 64 x 128 and 64 x 64 tiles).
+ * Those numbers only inform: explicit plans name the other kernels
+ * (w4a16_gemm_plan) and refuse them.  No reference counterpart.
+ */
+int w4a16_gemm_auto_plan(int64_t M, int64_t N, int64_t K, int64_t group_size, w4a16_plan* plan);
+
+/* Workspace bytes an automatic call of this shape can use (0 = none).  Less is
+ * enough where w4a16_gemm_plan's workspace_bytes says so: the call then takes
+ * fewer k-splits. */
 size_t w4a16_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t group_size);
 
 /*
@@ -191,6 +206,17 @@ int w4a16_gemm_f16_strided(const w4a16_plan* plan, const void* x, int64_t ldx,
  * that every GPU the library runs on holds until the process ends.
  */
 #define W4A16_NOALLOC_SCRATCH_BYTES (16u << 20)
+
+/*
+ * The automatic call with everything it takes: row strides as in
+ * w4a16_gemm_f16_strided, optional bias, and `flags` (W4A16_PLAN_ANY_ZEROS for
+ * zeros other than integers in [-1024, 1024], else 0; other bits are refused,
+ * W4A16_ERR_BAD_PLAN).
+ */
+int w4a16_gemm_f16_auto(const void* x, int64_t ldx, const int32_t* qweight, const void* scales,
+                        const void* zeros, const void* bias, void* y, int64_t ldy, int64_t M,
+                        int64_t N, int64_t K, int64_t group_size, int32_t flags, void* workspace,
+                        size_t workspace_bytes, void* stream);
 
 /*
  * As w4a16_gemm_f16_strided, for callers that cannot allocate device memory

@@ -1117,6 +1117,107 @@ int run_planned(const w4a16_plan* p, const void* x, int64_t ldx, const int32_t* 
   }
 }
 
+// ---- automatic calls on the one-wave-per-SIMD prefill kernel (gemm_wide.h) ----
+// Tiling and k-split by a cost model over its five tilings.  A workgroup takes
+// t0 + panels x tp us (panels of 64 k per wave), a CU holds one, and the time
+// grows with the share of the chip at work (its clock falls: `busy` x share in a
+// single round, a factor `rounds` per round beyond); a split adds its partials'
+// traffic and the reduction.  Fitted on MI355X at K = 4096 and 14336, N = 4096 /
+// 14336, M = 64 .. 4096, G = 128 (us: 256 x 256 tiles 75.4 / 243.5 for 64 / 224
+// panels on 56 / 16 CUs, 94.8 on 224, 104 a round at M = 4096; 128 x 256 49.5 /
+// 157.4, 57.2 on 224; 128 x 128 28.9 / 84.6, 33.1; 64 x 128 22.5 / 69.3, 24.7;
+// 64 x 64 13.7 / 38.0, 15.7).
+struct WideTiling {
+  int cfg, bm, bn, slices;
+  double t0, tp, busy, rounds;
+};
+constexpr WideTiling kWideTilings[] = {
+    {kWide256x256, 256, 256, 1, 8.2, 1.05, 0.30, 1.30},
+    {kWide128x256, 128, 256, 1, 6.3, 0.674, 0.18, 1.16},
+    {kWide128x128, 128, 128, 2, 6.6, 0.696, 0.12, 1.12},
+    {kWide64x128, 64, 128, 2, 3.8, 0.585, 0.07, 1.00},
+    {kWide64x64, 64, 64, 4, 4.0, 0.607, 0.17, 1.00},
+};
+// Half tiles' share of a round (the 256-row tiling's last one).
+constexpr double kWideHalfRound = 0.62;
+
+struct WideChoice {
+  int cfg, split;   // cfg kWideNone: not taken
+  double us;
+};
+
+// Partials beyond this are not asked for (w4a16_gemm_workspace_bytes).
+constexpr size_t kWideWorkspaceMax = 256u << 20;
+
+// The best tiling and split whose fp32 partials fit `max_bytes`.
+WideChoice wide_choice(int64_t M, int64_t N, int64_t K, bool any, int cus, size_t max_bytes) {
+  WideChoice best{kWideNone, 1, 0.0};
+  const int64_t panels = (K + 63) / 64;
+  for (const WideTiling& t : kWideTilings) {
+    if (any && t.cfg == kWide256x256) continue;
+    const int64_t tiles = (N + t.bn - 1) / t.bn * ((M + t.bm - 1) / t.bm);
+    const int max_split = t.cfg == kWide256x256 ? 1 : 16;
+    int last = 0;
+    for (int s = 1; s <= max_split; ++s) {
+      if (s > 1 && tiles * s > 2 * (int64_t)cus) break;
+      const int kts = wide_split_panels((int)K, s, t.slices);
+      const int ns = s > 1 ? (int)((panels + kts - 1) / kts) : 1;
+      if (ns == last || (s > 1 && ns < 2)) continue;
+      last = ns;
+      const uint64_t bytes = ns > 1 ? (uint64_t)ns * (uint64_t)M * (uint64_t)N * 4u : 0;
+      if (bytes > max_bytes) continue;
+      const int64_t wgs = tiles * ns;
+      const int64_t full = wgs / cus, rem = wgs % cus;
+      double us = t.t0 + t.tp * (double)(kts / t.slices);
+      if (full == 0 || (full == 1 && rem == 0)) {
+        us *= 1.0 + t.busy * (double)wgs / cus;
+      } else {
+        const bool halves = t.cfg == kWide256x256 && rem > 0 && 2 * rem <= cus;
+        us *= t.rounds * ((double)full + (rem == 0 ? 0.0 : halves ? kWideHalfRound : 1.0));
+      }
+      if (ns > 1) us += 1.8 + 0.25 * ns + ((double)bytes + 2.0 * (double)M * (double)N) / 5.0e6;
+      if (best.cfg == kWideNone || us < best.us) best = {t.cfg, ns, us};
+    }
+  }
+  return best;
+}
+
+// What the kernel needs of a call: 16-byte x rows, operands it can address, and
+// natural alignment of everything else.
+bool wide_operands_ok(const GemmArgs& a) {
+  return a.M > 0 && a.N > 0 && a.K > 0 && a.G % 32 == 0 && fits(a.M, a.N, a.K, a.G) &&
+         a.ldx % 8 == 0 && x_extent_bytes(a) < (1ull << 31) && aligned(a.x, 16) &&
+         aligned(a.qw, 4) && aligned(a.sc, 2) && aligned(a.zr, 2) && aligned(a.y, 2) &&
+         (!a.bias || aligned(a.bias, 2));
+}
+// Its vector form (whole column quads in one access each) or, else, the `any` one.
+bool wide_any(const GemmArgs& a) {
+  return !(a.N % 4 == 0 && a.ldy % 4 == 0 && aligned(a.qw, 16) && aligned(a.sc, 8) &&
+           aligned(a.zr, 8) && aligned(a.y, 8) && (!a.bias || aligned(a.bias, 8)));
+}
+bool scales_zeros_far(const GemmArgs& a) {
+  const uintptr_t sc = reinterpret_cast<uintptr_t>(a.sc), zr = reinterpret_cast<uintptr_t>(a.zr);
+  const uint64_t dist = sc < zr ? zr - sc : sc - zr;
+  return dist + (uint64_t)(a.K / a.G) * (uint64_t)a.N * 2u >= (1ull << 31);
+}
+
+// Whether an automatic call whose plan is `p` (auto_plan's: SIMT where operands
+// are not aligned for the vector kernels) takes the wide kernel: in place of
+//   * the streamed and register-tiled prefill kernels from M = 33 (measured on
+//     MI355X against them, us, G = 128: M = 64 / 128 / 256 / 512 / 1024 / 2048 /
+//     4096, K = 4096, N = 14336: 22.3 / 29.8 / 43.4 / 59.8 / 111 / 213 / 404 ->
+//     15.7 / 24.7 / 33.1 / 57.2 / 94.8 / 186 / 362; K = N = 4096, M = 128 / 256 /
+//     512 / 1024 / 4096 20.0 / 25.4 / 32.3 / 45.6 / 119 -> 14.2 / 15.6 / 24.7 /
+//     34.1 / 104), and of the 32-row streamed tiles where scales and zeros lie
+//     too far apart for their one buffer resource;
+//   * the SIMT kernel wherever the operands allow it (M = 93, K = 2080, N =
+//     1003, G = 32: 264 -> 27; M = 256, K = 4096, N = 1001 783 -> 41).
+bool wide_takes(const w4a16_plan& p, const GemmArgs& a) {
+  if (!wide_operands_ok(a)) return false;
+  if (p.kernel == W4A16_KERNEL_SIMT) return true;
+  return p.kernel == W4A16_KERNEL_MFMA && (a.M > 32 || (p.tile_cfg >= 11 && scales_zeros_far(a)));
+}
+
 // Automatic plan, falling back to the SIMT kernel when the pointers or row
 // strides do not meet the vector kernels' alignment.  Shape and strides must
 // have been checked.
@@ -1128,19 +1229,55 @@ int auto_plan(const void* x, int64_t ldx, const int32_t* qw, const void* sc, con
   const bool vec_aligned = aligned(x, 16) && aligned(qw, 16) && aligned(sc, 8) &&
                            aligned(zr, 8) && aligned(y, 8) && (!bias || aligned(bias, 8)) &&
                            strides_vec_ok(a, p->kernel, p->split_k);
-  if (p->kernel != W4A16_KERNEL_SIMT && !vec_aligned)
+  if (p->kernel != W4A16_KERNEL_SIMT && !vec_aligned) {
+    // the 16-column skinny blocks need no more than natural alignment
+    if (skinny_applicable(M, G) && fits(M, N, K, G) && M > 0 && N > 0 && K > 0 && aligned(x, 16) &&
+        aligned(qw, 4) && aligned(sc, 2) && aligned(zr, 2) &&
+        strides_vec_ok(a, W4A16_KERNEL_SKINNY, 1)) {
+      if (int st = make_plan(M, N, K, G, W4A16_KERNEL_SKINNY, 0, p)) return st;
+      p->tile_cfg = 0;
+      p->tile_m = (int32_t)((M + 15) / 16 * 16);
+      p->tile_n = 16;
+      p->grid_x = (N + 15) / 16;
+      return W4A16_OK;
+    }
     return make_plan(M, N, K, G, W4A16_KERNEL_SIMT, 0, p);
+  }
   return W4A16_OK;
+}
+
+// An automatic call with its plan `p` (flags set): the plan's kernel, or the wide
+// kernel where it takes the call.  Whatever the plan's own launch would refuse is
+// refused either way.
+int run_auto_plan(const w4a16_plan& p, const void* x, int64_t ldx, const int32_t* qw,
+                  const void* sc, const void* zr, const void* bias, void* y, int64_t ldy,
+                  int64_t M, int64_t N, int64_t K, int64_t G, void* ws, size_t ws_bytes,
+                  void* stream) {
+  const GemmArgs a{x, qw, sc, zr, bias, y, (int)M, (int)N, (int)K, (int)G, (int)ldx, (int)ldy,
+                   (p.flags & W4A16_PLAN_ANY_ZEROS) != 0};
+  const bool ws_ok = ws && aligned(ws, 256);
+  const size_t need = p.split_k > 1 ? (size_t)p.workspace_bytes : 0;
+  if (x && qw && sc && zr && y && !(p.flags & ~W4A16_PLAN_ANY_ZEROS) &&
+      (need == 0 || (ws_ok && ws_bytes >= need)) && wide_takes(p, a)) {
+    const int cus = device_cu_count();
+    const bool any = wide_any(a);
+    const WideChoice w = wide_choice(M, N, K, any, cus, ws_ok ? ws_bytes : 0);
+    if (w.cfg != kWideNone)
+      return to_status(launch_wide(a, w.cfg, any, w.split, static_cast<float*>(ws), cus,
+                                   static_cast<hipStream_t>(stream)));
+  }
+  return run_planned(&p, x, ldx, qw, sc, zr, bias, y, ldy, M, N, K, G, ws, ws_bytes, stream);
 }
 
 int run_auto(const void* x, int64_t ldx, const int32_t* qw, const void* sc, const void* zr,
              const void* bias, void* y, int64_t ldy, int64_t M, int64_t N, int64_t K, int64_t G,
-             void* ws, size_t ws_bytes, void* stream) {
+             int32_t flags, void* ws, size_t ws_bytes, void* stream) {
   if (int st = check_gemm_shape(M, N, K, G)) return st;
   if (int st = check_strides(M, N, K, ldx, ldy)) return st;
   w4a16_plan p;
   if (int st = auto_plan(x, ldx, qw, sc, zr, bias, y, ldy, M, N, K, G, &p)) return st;
-  return run_planned(&p, x, ldx, qw, sc, zr, bias, y, ldy, M, N, K, G, ws, ws_bytes, stream);
+  p.flags = flags;
+  return run_auto_plan(p, x, ldx, qw, sc, zr, bias, y, ldy, M, N, K, G, ws, ws_bytes, stream);
 }
 
 // Split-K partial bytes a plan's kernels write (what run_planned requires of
@@ -1236,13 +1373,46 @@ size_t w4a16_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t group
   w4a16_plan p;
   if (check_gemm_shape(M, N, K, group_size) != W4A16_OK) return 0;
   if (make_plan(M, N, K, group_size, W4A16_KERNEL_AUTO, 0, &p) != W4A16_OK) return 0;
-  return (size_t)p.workspace_bytes;
+  size_t bytes = (size_t)p.workspace_bytes;
+  // the wide kernel's splits: where the plan is a prefill one it may replace, and
+  // where odd widths or alignment send the call to it
+  if (group_size % 32 == 0 && M > 0 && N > 0 && K > 0 && fits(M, N, K, group_size) &&
+      (p.kernel == W4A16_KERNEL_MFMA || p.kernel == W4A16_KERNEL_SIMT)) {
+    const WideChoice w = wide_choice(M, N, K, N % 4 != 0, device_cu_count(), kWideWorkspaceMax);
+    if (w.split > 1) {
+      const size_t need = (size_t)w.split * (size_t)M * (size_t)N * 4u;
+      if (need > bytes) bytes = need;
+    }
+  }
+  return bytes;
+}
+
+int w4a16_gemm_auto_plan(int64_t M, int64_t N, int64_t K, int64_t group_size, w4a16_plan* plan) {
+  if (int st = w4a16_gemm_plan(M, N, K, group_size, W4A16_KERNEL_AUTO, 0, plan)) return st;
+  const bool wide = M > 0 && N > 0 && K > 0 && group_size % 32 == 0 && fits(M, N, K, group_size) &&
+                    ((plan->kernel == W4A16_KERNEL_MFMA && M > 32) ||
+                     plan->kernel == W4A16_KERNEL_SIMT);
+  if (!wide) return W4A16_OK;
+  const WideChoice w = wide_choice(M, N, K, N % 4 != 0, device_cu_count(),
+                                   w4a16_gemm_workspace_bytes(M, N, K, group_size));
+  for (const WideTiling& t : kWideTilings)
+    if (t.cfg == w.cfg) {
+      plan->kernel = W4A16_KERNEL_MFMA;
+      plan->tile_cfg = t.cfg;
+      plan->tile_m = t.bm;
+      plan->tile_n = t.bn;
+      plan->split_k = w.split;
+      plan->grid_x = (N + t.bn - 1) / t.bn * ((M + t.bm - 1) / t.bm) * w.split;
+      plan->grid_y = 1;
+      plan->workspace_bytes = w.split > 1 ? w.split * M * N * 4 : 0;
+    }
+  return W4A16_OK;
 }
 
 int w4a16_gemm_f16(const void* x, const int32_t* qweight, const void* scales, const void* zeros,
                    void* y, int64_t M, int64_t N, int64_t K, int64_t group_size,
                    void* workspace, size_t workspace_bytes, void* stream) {
-  return run_auto(x, K, qweight, scales, zeros, nullptr, y, N, M, N, K, group_size, workspace,
+  return run_auto(x, K, qweight, scales, zeros, nullptr, y, N, M, N, K, group_size, 0, workspace,
                   workspace_bytes, stream);
 }
 
@@ -1250,7 +1420,7 @@ int w4a16_linear_f16(const void* x, const int32_t* qweight, const void* scales,
                      const void* zeros, const void* bias, void* y, int64_t M, int64_t N,
                      int64_t K, int64_t group_size, void* workspace, size_t workspace_bytes,
                      void* stream) {
-  return run_auto(x, K, qweight, scales, zeros, bias, y, N, M, N, K, group_size, workspace,
+  return run_auto(x, K, qweight, scales, zeros, bias, y, N, M, N, K, group_size, 0, workspace,
                   workspace_bytes, stream);
 }
 
@@ -1268,10 +1438,19 @@ int w4a16_gemm_f16_strided(const w4a16_plan* plan, const void* x, int64_t ldx,
                            int64_t group_size, void* workspace, size_t workspace_bytes,
                            void* stream) {
   if (!plan)
-    return run_auto(x, ldx, qweight, scales, zeros, bias, y, ldy, M, N, K, group_size, workspace,
+    return run_auto(x, ldx, qweight, scales, zeros, bias, y, ldy, M, N, K, group_size, 0, workspace,
                     workspace_bytes, stream);
   return run_planned(plan, x, ldx, qweight, scales, zeros, bias, y, ldy, M, N, K, group_size,
                      workspace, workspace_bytes, stream);
+}
+
+int w4a16_gemm_f16_auto(const void* x, int64_t ldx, const int32_t* qweight, const void* scales,
+                        const void* zeros, const void* bias, void* y, int64_t ldy, int64_t M,
+                        int64_t N, int64_t K, int64_t group_size, int32_t flags, void* workspace,
+                        size_t workspace_bytes, void* stream) {
+  if (flags & ~W4A16_PLAN_ANY_ZEROS) return W4A16_ERR_BAD_PLAN;
+  return run_auto(x, ldx, qweight, scales, zeros, bias, y, ldy, M, N, K, group_size, flags,
+                  workspace, workspace_bytes, stream);
 }
 
 int w4a16_gemm_f16_noalloc(const w4a16_plan* plan, const void* x, int64_t ldx,

@@ -297,6 +297,22 @@ __global__ __launch_bounds__(256) void splitk_reduce(const float* __restrict__ p
   *reinterpret_cast<f16x4*>(Y + row * (size_t)ldy + col) = o;
 }
 
+// One element a thread: N % 4 != 0, or y off the quad's alignment.
+__global__ __launch_bounds__(256) void splitk_reduce_any(const float* __restrict__ part,
+                                                         const f16* __restrict__ bias,
+                                                         f16* __restrict__ Y, int M, int N,
+                                                         int ldy, int S) {
+  const size_t n = (size_t)M * N, e = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (e >= n) return;
+  float s = part[e];
+  for (int i = 1; i < S; ++i) s += part[(size_t)i * n + e];
+  const size_t row = e / (size_t)N;
+  const int col = (int)(e - row * (size_t)N);
+  f16 o = f32_to_f16(s);
+  if (bias) o = o + bias[col];
+  Y[row * (size_t)ldy + col] = o;
+}
+
 template <int WAVES_M, int WAVES_N, bool G64, bool AZ>
 hipError_t launch_wgz(const GemmArgs& a, int split, float* part, hipStream_t st) {
   constexpr int BM = 16 * kMT * WAVES_M;
@@ -332,6 +348,12 @@ bool occ2_gemm_applicable(int M, int N, int K, int G) {
 
 hipError_t launch_splitk_reduce(const float* part, const void* bias, void* y, int M, int N, int ldy,
                                 int S, hipStream_t st) {
+  if (N % 4 != 0 || ldy % 4 != 0 || (reinterpret_cast<uintptr_t>(y) & 7) != 0) {
+    const size_t n = (size_t)M * (size_t)N;
+    hipLaunchKernelGGL(splitk_reduce_any, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, part,
+                       static_cast<const f16*>(bias), static_cast<f16*>(y), M, N, ldy, S);
+    return hipGetLastError();
+  }
   const size_t nq = (size_t)M * (size_t)(N / 4);
   hipLaunchKernelGGL(splitk_reduce, dim3((unsigned)((nq + 255) / 256)), dim3(256), 0, st, part,
                      static_cast<const f16*>(bias), static_cast<f16*>(y), M, N, ldy, S);

@@ -83,8 +83,8 @@ bool mfma_cfg_splits(int cfg);
 // split > 1 (cfg 7, 11-13 only): fp32 partials in `part`, occ2_workspace_bytes().
 hipError_t launch_mfma(const GemmArgs& a, int cfg, int split, float* part, hipStream_t st);
 // Split-K epilogue shared by the GEMV and the prefill kernels: y[M, N] =
-// fp16(sum of the S fp32 partials [S][M][N], in split order) (+ fp16 bias).
-// N % 4 == 0.
+// fp16(sum of the S fp32 partials [S][M][N], in split order) (+ fp16 bias); any
+// N and alignment (four columns a thread where both allow it).
 hipError_t launch_splitk_reduce(const float* part, const void* bias, void* y, int M, int N, int ldy,
                                 int S, hipStream_t st);
 // Two-waves-per-SIMD 16x16x32 kernel (mfma cfg 7: 128 x 256): needs K % 64 == 0.
@@ -105,6 +105,23 @@ int stream_splits(int K, int split, int slices = 1);
 hipError_t launch_stream_gemm(const GemmArgs& a, int rows, int split, float* part,
                               hipStream_t st, int slices = 1);
 hipError_t launch_occ2_gemm(const GemmArgs& a, int split, float* part, hipStream_t st);
+
+// One-wave-per-SIMD prefill kernel (gemm_wide.h): tilings of automatic calls
+// only (no plan names them).  `any`: N % 4 != 0 or less alignment than the
+// vector form needs; not on the 256-row tiles.  split > 1: fp32 partials
+// [split][M][N] in `part`, then the reduction.
+enum WideConfig {
+  kWideNone = 0,
+  kWide256x256 = 16,   // tile_cfg numbers in what w4a16_gemm_auto_plan reports
+  kWide128x256 = 17,
+  kWide128x128 = 18,   // two k-slices per workgroup
+  kWide64x128 = 19,    // two
+  kWide64x64 = 20      // four
+};
+// 64-k panels per split (whole 4-panel blocks per slice).
+int wide_split_panels(int K, int split, int slices);
+hipError_t launch_wide(const GemmArgs& a, int cfg, bool any, int split, float* part, int cus,
+                       hipStream_t st);
 
 // Buffer-addressed kernels need every operand below 2 GiB.
 bool operands_fit(int M, int N, int K, int G);

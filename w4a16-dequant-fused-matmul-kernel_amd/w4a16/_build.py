@@ -20,8 +20,9 @@ CSRC = os.path.join(ROOT_DIR, "csrc")
 BUILD_DIR = os.path.join(CSRC, "_build")
 LIB_PATH = os.path.join(PKG_DIR, "libw4a16.so")
 SOURCES = ["gemv.hip", "gemm_mfma.hip", "gemm_occ2.hip", "gemm_stream.hip", "gemm_skinny.hip",
-           "simt.hip", "quant.hip", "capi.cpp"]
-HEADERS = ["w4a16_device.h", "w4a16_launch.h", "decode_table.inc"]
+           "gemm_wide_256.hip", "gemm_wide_128.hip", "gemm_wide_64.hip", "simt.hip", "quant.hip",
+           "capi.cpp"]
+HEADERS = ["w4a16_device.h", "w4a16_launch.h", "gemm_wide.h", "decode_table.inc"]
 PUBLIC_HEADER = os.path.join(os.path.dirname(ROOT_DIR), "include", "w4a16.h")
 ARCH = "gfx950"
 
@@ -61,6 +62,9 @@ SOURCE_FLAGS = {
     "gemv.hip": _PRELOAD,
     "gemm_skinny.hip": _PRELOAD,
     "gemm_stream.hip": _PRELOAD,
+    "gemm_wide_256.hip": _PRELOAD,
+    "gemm_wide_128.hip": _PRELOAD,
+    "gemm_wide_64.hip": _PRELOAD,
     "gemm_occ2.hip": _PRELOAD,   # and the split-K reduction kernel
 }
 

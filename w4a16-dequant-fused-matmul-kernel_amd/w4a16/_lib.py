@@ -79,6 +79,7 @@ SIGNATURES = {
     "w4a16_build_id": (ctypes.c_char_p, []),
     "w4a16_status_string": (ctypes.c_char_p, [_int]),
     "w4a16_gemm_plan": (_int, [_i64, _i64, _i64, _i64, _i32, _i32, ctypes.POINTER(Plan)]),
+    "w4a16_gemm_auto_plan": (_int, [_i64, _i64, _i64, _i64, ctypes.POINTER(Plan)]),
     "w4a16_gemm_workspace_bytes": (_sz, [_i64, _i64, _i64, _i64]),
     "w4a16_zeros_check_f16": (_int, [_vp, _i64, _vp, _vp]),
     "w4a16_gemm_f16": (_int, [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp, _sz, _vp]),
@@ -92,6 +93,10 @@ SIGNATURES = {
         _int,
         [ctypes.POINTER(Plan), _vp, _i64, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64,
          _vp, _sz, _vp],
+    ),
+    "w4a16_gemm_f16_auto": (
+        _int,
+        [_vp, _i64, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i32, _vp, _sz, _vp],
     ),
     "w4a16_gemm_f16_noalloc": (
         _int,
@@ -174,4 +179,12 @@ def plan(M: int, N: int, K: int, group_size: int, kernel: int = 0, split_k: int 
     p = Plan()
     check(load().w4a16_gemm_plan(M, N, K, group_size, kernel, split_k, ctypes.byref(p)),
           "w4a16_gemm_plan")
+    return p
+
+
+def auto_plan(M: int, N: int, K: int, group_size: int) -> Plan:
+    """What an automatic call runs for this shape (see w4a16_gemm_auto_plan)."""
+    p = Plan()
+    check(load().w4a16_gemm_auto_plan(M, N, K, group_size, ctypes.byref(p)),
+          "w4a16_gemm_auto_plan")
     return p

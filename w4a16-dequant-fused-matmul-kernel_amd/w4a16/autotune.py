@@ -76,8 +76,9 @@ def _plan_from(fields: dict) -> _lib.Plan:
 
 
 def candidates(M: int, N: int, K: int, G: int) -> list[tuple[str, _lib.Plan]]:
-    """The static plan first, then every other plan the library has for the
-    shape: GEMV column widths, wave counts, staging and MFMA-dot forms and
+    """The static plan first, then the automatic call (a plan naming no kernel:
+    prefill shapes run one no plan names) and every other plan the library has
+    for the shape: GEMV column widths, wave counts, staging and MFMA-dot forms and
     k-splits (M <= 8); skinny block widths and row groups (M <= 64); streamed
     prefill tiles (32 / 64 / 128 rows, one or two k-slices) and their k-splits,
     and the register-staged tilings where K % 256 != 0.  Plans a shape cannot
@@ -100,6 +101,7 @@ def candidates(M: int, N: int, K: int, G: int) -> list[tuple[str, _lib.Plan]]:
     add("static", _lib.plan(M, N, K, G))
     if M == 0 or N == 0 or K == 0:
         return out
+    add("automatic", _lib.Plan())   # kernel AUTO: the automatic call
     if M <= 8 and N % 4 == 0 and G % 32 == 0:
         # column blocks that leave at least an eighth of the CUs a block;
         # k-splits 2 and 4 (8 from K = 16384)
@@ -156,7 +158,13 @@ def time_plans(x, qweight, scales, zeros, G: int, plans, reps: int = 3,
     The output is a scratch tensor with row stride `ldy` (default N), so a plan
     is tried on the caller's layout.  A plan the library refuses gets +inf.
     Each repetition is a run of calls of about `budget_us`."""
-    from .hip_kernel import w4a16_matmul_planned
+    from .hip_kernel import w4a16_matmul_planned, w4a16_matmul_untuned
+
+    def call(p):
+        if p.kernel == _lib.KERNEL_AUTO:
+            w4a16_matmul_untuned(x, qweight, scales, zeros, G, y)
+        else:
+            w4a16_matmul_planned(x, qweight, scales, zeros, G, p, out=y)
 
     M, K = x.shape
     N = qweight.shape[1]
@@ -167,10 +175,10 @@ def time_plans(x, qweight, scales, zeros, G: int, plans, reps: int = 3,
     for p in plans:
         try:
             for _ in range(2):
-                w4a16_matmul_planned(x, qweight, scales, zeros, G, p, out=y)
+                call(p)
             t0, t1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
             t0.record(stream)
-            w4a16_matmul_planned(x, qweight, scales, zeros, G, p, out=y)
+            call(p)
             t1.record(stream)
             t1.synchronize()
             live.append(True)
@@ -187,7 +195,7 @@ def time_plans(x, qweight, scales, zeros, G: int, plans, reps: int = 3,
             t0, t1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
             t0.record(stream)
             for _ in range(n):
-                w4a16_matmul_planned(x, qweight, scales, zeros, G, p, out=y)
+                call(p)
             t1.record(stream)
             t1.synchronize()
             times[i].append(t0.elapsed_time(t1) * 1e3 / n)
@@ -233,13 +241,14 @@ def _key(x, M, N, K, G, ldx, ldy, any_zeros) -> str:
 def plan_for_call(x, qweight, scales, zeros, G: int, M: int, N: int, K: int, ldx: int, ldy: int,
                   any_zeros: bool):
     """The tuned plan of this call's shape (tuning it now if it is new), or None
-    under graph capture when the shape has not been tuned."""
+    where the automatic call is the fastest, and under graph capture when the
+    shape has not been tuned."""
     key = _key(x, M, N, K, G, ldx, ldy, any_zeros)
     with _LOCK:
         _load_file()
         hit = _CACHE.get(key)
     if hit is not None:
-        return _plan_from(hit["plan"])
+        return _named(_plan_from(hit["plan"]))
     if torch.cuda.is_current_stream_capturing():
         return None
     cands = candidates(M, N, K, G)
@@ -251,4 +260,8 @@ def plan_for_call(x, qweight, scales, zeros, G: int, M: int, N: int, K: int, ldx
     with _LOCK:
         _CACHE[key] = entry
         _save_file()
-    return _plan_from(entry["plan"])
+    return _named(_plan_from(entry["plan"]))
+
+
+def _named(p: _lib.Plan) -> "_lib.Plan | None":
+    return None if p.kernel == _lib.KERNEL_AUTO else p

@@ -10,10 +10,12 @@ kernel is chosen inside ``libw4a16.so`` by shape:
   workgroup, split-K only when N is too narrow;
 * other M <= 64 on small weights: skinny GEMM on v_mfma_f32_16x16x32_f16, 16
   columns per workgroup over the whole of K;
-* 4 <= M <= 64 on larger weights, and M > 64: the streamed prefill GEMM on
-  MFMA (32-, 64- or 128-row tiles, split along K where the tiles are few);
-* shapes the vector kernels do not take (N % 4 != 0 beyond the skinny range,
-  G % 32 != 0, misaligned views, operands >= 2 GiB): the sequential-k SIMT
+* 4 <= M <= 32 on larger weights: the streamed GEMM on MFMA (32-row tiles,
+  split along K where the tiles are few);
+* larger M, any N, and operands less aligned than the kernels above need: the
+  one-wave-per-SIMD prefill GEMM on MFMA (64 to 256-row tiles, k-slices in the
+  workgroup and splits across workgroups where the tiles are few);
+* what is left (x rows off 16 bytes, operands >= 2 GiB): the sequential-k SIMT
   kernel.
 
 Row-strided views (inner stride 1, row stride >= the row length) are accepted
@@ -127,10 +129,10 @@ _FAR_SZ_WARNED = False
 
 
 def _warn_far_scales_zeros(scales: Tensor, zeros: Tensor, M: int) -> None:
-    """Warn once per process when scales and zeros lie 2 GiB or more apart:
-    the streamed MFMA kernels (prefill, and small batches on large weights)
-    reach both through one buffer resource, so such calls run the
-    register-tiled kernel instead -- same results, slower."""
+    """Warn once per process when a planned call's scales and zeros lie 2 GiB or
+    more apart: the streamed MFMA kernels reach both through one buffer
+    resource, so such plans run the register-tiled kernel instead -- same
+    results, slower."""
     global _FAR_SZ_WARNED
     if _FAR_SZ_WARNED or M < 4:
         return
@@ -145,39 +147,37 @@ def _warn_far_scales_zeros(scales: Tensor, zeros: Tensor, M: int) -> None:
             RuntimeWarning, stacklevel=4)
 
 
-def _launch(x, qweight, scales, zeros, bias, y, M, N, K, G, plan: "_lib.Plan | None"):
+def _launch(x, qweight, scales, zeros, bias, y, M, N, K, G, plan: "_lib.Plan | None",
+            tune: bool = True):
     dev = x.device
-    _warn_far_scales_zeros(scales, zeros, M)
+    if plan is not None:   # an automatic call takes a kernel that does not mind
+        _warn_far_scales_zeros(scales, zeros, M)
     with rt.on_device(dev):
         any_zeros = zeros_need_any_form(zeros)
-        if plan is None and autotune.enabled():
+        if plan is None and tune and autotune.enabled():
             plan = autotune.plan_for_call(x, qweight, scales, zeros, G, M, N, K, _row_stride(x),
                                           _row_stride(y), any_zeros)
-        if any_zeros:
+        if any_zeros and plan is not None:
             # the any-zero kernels, through a plan carrying the flag
-            if plan is None:
-                plan = _lib.plan(M, N, K, G)
-            else:
-                plan = _lib.Plan.from_buffer_copy(plan)
+            plan = _lib.Plan.from_buffer_copy(plan)
             plan.flags |= _lib.PLAN_ANY_ZEROS
-        if plan is None:
-            ws_bytes = rt.lib().w4a16_gemm_workspace_bytes(M, N, K, G)
-        else:
-            ws_bytes = int(plan.workspace_bytes)
+        ws_bytes = (rt.lib().w4a16_gemm_workspace_bytes(M, N, K, G) if plan is None
+                    else int(plan.workspace_bytes))
         ws = rt.workspace(dev, ws_bytes)
         stream = rt.stream_ptr(dev)
         ldx, ldy = _row_stride(x), _row_stride(y)
-        if ldx != K or ldy != N:
+        if plan is None:
+            code = rt.lib().w4a16_gemm_f16_auto(
+                x.data_ptr(), ldx, qweight.data_ptr(), scales.data_ptr(), zeros.data_ptr(),
+                rt.ptr(bias), y.data_ptr(), ldy, M, N, K, G,
+                _lib.PLAN_ANY_ZEROS if any_zeros else 0, rt.ptr(ws),
+                0 if ws is None else ws.numel(), stream)
+        elif ldx != K or ldy != N:
             code = rt.lib().w4a16_gemm_f16_strided(
-                None if plan is None else ctypes.byref(plan), x.data_ptr(), ldx,
+                ctypes.byref(plan), x.data_ptr(), ldx,
                 qweight.data_ptr(), scales.data_ptr(), zeros.data_ptr(), rt.ptr(bias),
                 y.data_ptr(), ldy, M, N, K, G, rt.ptr(ws), 0 if ws is None else ws.numel(),
                 stream)
-        elif plan is None:
-            code = rt.lib().w4a16_linear_f16(
-                x.data_ptr(), qweight.data_ptr(), scales.data_ptr(), zeros.data_ptr(),
-                rt.ptr(bias), y.data_ptr(), M, N, K, G, rt.ptr(ws),
-                0 if ws is None else ws.numel(), stream)
         else:
             code = rt.lib().w4a16_gemm_f16_planned(
                 ctypes.byref(plan), x.data_ptr(), qweight.data_ptr(), scales.data_ptr(),
@@ -252,3 +252,11 @@ def w4a16_matmul_planned(x: Tensor, qweight: Tensor, scales: Tensor, zeros: Tens
     M, K, N = _check_operands(x, qweight, scales, zeros, group_size)
     y = _output(x, M, N, out)
     return _launch(x, qweight, scales, zeros, bias, y, M, N, K, group_size, plan)
+
+
+def w4a16_matmul_untuned(x: Tensor, qweight: Tensor, scales: Tensor, zeros: Tensor,
+                         group_size: int, out: Tensor) -> Tensor:
+    """The automatic call, whether or not autotuning is on (the tuner's own)."""
+    M, K, N = _check_operands(x, qweight, scales, zeros, group_size)
+    y = _output(x, M, N, out)
+    return _launch(x, qweight, scales, zeros, None, y, M, N, K, group_size, None, tune=False)
