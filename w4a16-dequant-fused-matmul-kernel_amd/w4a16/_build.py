@@ -103,13 +103,62 @@ def _link(objs: list[str], path: str, verbose: bool) -> None:
     os.replace(tmp, path)
 
 
+NATIVE_SOURCE = "native.cpp"
+NATIVE_PATH = os.path.join(PKG_DIR, "_native.so")
+
+
+def native_hash() -> str:
+    """Like source_hash(), for the CPython module _native.so: its source, the
+    public header, and the torch and Python versions it is compiled against."""
+    import torch
+
+    h = hashlib.sha256()
+    for path in (os.path.join(CSRC, NATIVE_SOURCE), PUBLIC_HEADER):
+        with open(path, "rb") as f:
+            h.update(f.read())
+    h.update(f"{torch.__version__} {sys.version_info[:2]}".encode())
+    return h.hexdigest()
+
+
+def build_native(verbose: bool = False) -> str:
+    """Compile _native.so (host code only, against torch's headers)."""
+    import sysconfig
+
+    import torch
+
+    root = os.path.dirname(torch.__file__)
+    rocm = os.path.dirname(os.path.dirname(os.path.realpath(hipcc())))
+    tmp = NATIVE_PATH + ".tmp"
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f'-DW4A16_NATIVE_HASH="{native_hash()}"',
+           *(f"-isystem{p}" for p in (os.path.join(root, "include"),
+                                      os.path.join(root, "include", "torch", "csrc", "api",
+                                                   "include"),
+                                      os.path.join(rocm, "include"), "/opt/rocm/include",
+                                      sysconfig.get_paths()["include"])),
+           os.path.join(CSRC, NATIVE_SOURCE), "-o", tmp, "-L" + os.path.join(root, "lib"),
+           "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip", "-ldl"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"g++ failed on {NATIVE_SOURCE}:\n{res.stdout}\n{res.stderr}")
+    os.replace(tmp, NATIVE_PATH)
+    return NATIVE_PATH
+
+
 def build(verbose: bool = False, jobs: int | None = None) -> str:
-    """Compile every source and link libw4a16.so; returns the library path."""
+    """Compile every source, link libw4a16.so and compile _native.so; returns the
+    library path."""
     os.makedirs(BUILD_DIR, exist_ok=True)
     jobs = jobs or min(len(SOURCES), os.cpu_count() or 1, 8)
     defines = [f'-DW4A16_SOURCE_HASH="{source_hash()}"']
     with ThreadPoolExecutor(max_workers=jobs) as ex:
+        native = ex.submit(build_native, verbose)
         objs = list(ex.map(lambda s: _compile(s, verbose, defines), SOURCES))
+        native.result()
     _link(objs, LIB_PATH, verbose)
     return LIB_PATH
 

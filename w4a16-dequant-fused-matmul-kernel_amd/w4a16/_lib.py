@@ -162,6 +162,24 @@ def load() -> ctypes.CDLL:
         return lib
 
 
+def load_native(zeros_key: str):
+    """The CPython module ``_native`` (csrc/native.cpp), bound to the loaded
+    library; ImportError if it is missing, stale or was built for another torch."""
+    load()
+    from . import _build
+
+    how = "build it with `python -m w4a16._build`"
+    try:
+        from . import _native
+    except ImportError as e:
+        raise ImportError(f"cannot import {_build.NATIVE_PATH}: {e}; {how}") from e
+    if os.path.isdir(_build.CSRC) and _native.build_id() != _build.native_hash():
+        raise ImportError(f"{_build.NATIVE_PATH} was built from other sources or for another "
+                          f"torch; {how}")
+    _native.init(LIB_PATH, zeros_key)
+    return _native
+
+
 def status_text(code: int) -> str:
     lib = load()
     return lib.w4a16_status_string(code).decode()

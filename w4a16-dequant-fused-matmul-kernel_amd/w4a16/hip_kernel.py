@@ -195,6 +195,28 @@ def _output(x: Tensor, M: int, N: int, out: Tensor | None) -> Tensor:
     return out
 
 
+def _native_gemm(x, *rest):
+    """The automatic call in one C function (csrc/native.cpp): y, or None where
+    the checks and the launch below have to run.  This loads it on the first
+    call with device operands and takes its place."""
+    global _native_gemm
+    if not (isinstance(x, Tensor) and x.is_cuda):
+        return None
+    fn = _lib.load_native(_ZKEY).gemm
+    _native_gemm = fn
+    return fn(x, *rest)
+
+
+def linear_native(x: Tensor, qweight, scales, zeros, bias, group_size: int, in_features: int,
+                  out_features: int) -> Tensor | None:
+    """W4A16Linear.forward's whole computation, x of any leading dimensions; None
+    where the module has to go through its own checks and w4a16_linear."""
+    if autotune.enabled():
+        return None
+    return _native_gemm(x, qweight, scales, zeros, bias, group_size, None, in_features,
+                        out_features)
+
+
 def w4a16_matmul(
     x: Tensor,
     qweight: Tensor,
@@ -214,6 +236,10 @@ def w4a16_matmul(
     Returns:
         fp16 [M, N], fp32-accumulated.
     """
+    if not autotune.enabled():
+        y = _native_gemm(x, qweight, scales, zeros, None, group_size, out, None, None)
+        if y is not None:
+            return y
     M, K, N = _check_operands(x, qweight, scales, zeros, group_size)
     y = _output(x, M, N, out)
     return _launch(x, qweight, scales, zeros, None, y, M, N, K, group_size, None)
@@ -227,6 +253,10 @@ def w4a16_linear(x: Tensor, qweight: Tensor, scales: Tensor, zeros: Tensor,
     (linear.py:89-91): the GEMM result is rounded to fp16, then the fp16 bias is
     added with one more fp16 rounding.
     """
+    if not autotune.enabled():
+        y = _native_gemm(x, qweight, scales, zeros, bias, group_size, out, None, None)
+        if y is not None:
+            return y
     M, K, N = _check_operands(x, qweight, scales, zeros, group_size)
     if bias is not None:
         assert bias.shape == (N,) and bias.dtype == torch.float16 and bias.is_contiguous()

@@ -18,8 +18,8 @@ from __future__ import annotations
 import torch
 from torch import Tensor, nn
 
-from .hip_kernel import mark_integer_zeros, w4a16_linear
-from .quant import quantize_weight
+from .hip_kernel import linear_native, mark_integer_zeros, w4a16_linear
+from .quant import quantize_finish, quantize_start, quantize_weight
 
 __all__ = ["W4A16Linear"]
 
@@ -93,11 +93,18 @@ class W4A16Linear(nn.Module):
                 layer.bias.copy_(linear.bias.detach().to(torch.float16))
             return layer
         # a fresh layer takes the quantiser's tensors as its buffers: nothing is
-        # zeroed first or copied afterwards
-        layer = cls(in_features, out_features, group_size=group_size, bias=has_bias, device="meta")
-        layer.qweight, layer.scales, layer.zeros = quantize_weight(W, group_size)
-        if has_bias:
-            layer.bias = linear.bias.detach().to(W.device, torch.float16, copy=True).contiguous()
+        # zeroed first or copied afterwards; it is made while the kernel runs
+        _check_sizes(in_features, group_size)
+        started = quantize_start(W, group_size)
+        try:
+            layer = cls(in_features, out_features, group_size=group_size, bias=has_bias,
+                        device="meta")
+            if has_bias:
+                layer.bias = linear.bias.detach().to(W.device, torch.float16,
+                                                     copy=True).contiguous()
+        finally:
+            packed = quantize_finish(started)
+        layer.qweight, layer.scales, layer.zeros = packed
         return layer
 
     def quantize_from_dense(self, W: Tensor) -> None:
@@ -116,6 +123,15 @@ class W4A16Linear(nn.Module):
     def forward(self, x: Tensor) -> Tensor:
         """``fp16(x @ dequant(W)) + bias`` over the last dimension of ``x``
         (reference linear.py:82-92); leading dimensions are kept."""
+        if type(self) is W4A16Linear:
+            # the buffers straight from their dict: nn.Module's attribute lookup
+            # costs 2 us for the four
+            b = self._buffers
+            y = linear_native(x, b.get("qweight"), b.get("scales"), b.get("zeros"),
+                              b["bias"] if "bias" in b else self.bias, self.group_size,
+                              self.in_features, self.out_features)
+            if y is not None:
+                return y
         if x.dtype != torch.float16:
             raise AssertionError(f"W4A16Linear expects fp16 activations, got {x.dtype}")
         if x.shape[-1] != self.in_features:

@@ -107,6 +107,12 @@ def quantize_weight(W: Tensor, group_size: int = 128) -> tuple[Tensor, Tensor, T
     Returns:
         (qweight int32 [K//8, N], scales fp16 [K//G, N], zeros fp16 [K//G, N])
     """
+    return quantize_finish(quantize_start(W, group_size))
+
+
+def quantize_start(W: Tensor, group_size: int) -> tuple:
+    """quantize_weight up to its launch; the result goes to quantize_finish, in
+    the same thread with the same current stream, whatever happens in between."""
     assert W.dim() == 2, f"quantize_weight expects 2D [K, N], got {tuple(W.shape)}"
     K, N = W.shape
     if K % _NIBBLES_PER_INT32 != 0:
@@ -115,6 +121,7 @@ def quantize_weight(W: Tensor, group_size: int = 128) -> tuple[Tensor, Tensor, T
         raise ValueError(f"K={K} must be divisible by group_size={group_size}")
     G = group_size
     home, dev, (Wd,) = rt.stage_to_device(W.detach())
+    flag = None
     with rt.on_device(dev):
         if Wd.dtype not in (torch.float16, torch.float32):
             Wd = Wd.to(torch.float32)
@@ -122,11 +129,23 @@ def quantize_weight(W: Tensor, group_size: int = 128) -> tuple[Tensor, Tensor, T
         scales = torch.empty((K // G, N), dtype=torch.float16, device=dev)
         zeros = torch.empty((K // G, N), dtype=torch.float16, device=dev)
         if Wd.numel():
-            flag = _flag(dev)
+            # The kernel sets the flag only for a non-finite weight, so it lies in
+            # pinned host memory: no fill kernel before, no copy back after, only
+            # the wait (quantising 4096 x 14336: 63.5 -> 60.5 us; from_linear,
+            # whose module is built meanwhile: 98.5 -> 74.3 us at 4096 x 11008).
+            flag = torch.empty(1, dtype=torch.int32, device="cpu", pin_memory=True)
+            flag[0] = 0
             _lib.check(_quantize_pack(Wd, qweight, scales, zeros, G, flag), "w4a16_quantize_pack")
-            if int(flag.item()) != 0:
-                raise AssertionError(
-                    "uint4 values must be in [0,15]: W holds a non-finite value")
+    return home, dev, flag, qweight, scales, zeros, Wd
+
+
+def quantize_finish(started: tuple) -> tuple[Tensor, Tensor, Tensor]:
+    """Wait for quantize_start's kernel, check its flag, return the results."""
+    home, dev, flag, qweight, scales, zeros, _ = started
+    if flag is not None:
+        torch.cuda.current_stream(dev).synchronize()
+        if flag.item() != 0:
+            raise AssertionError("uint4 values must be in [0,15]: W holds a non-finite value")
     zeros = zeros.to(home)
     mark_integer_zeros(zeros)   # zero-points 0..15: the integer-zero kernels take them
     return qweight.to(home), scales.to(home), zeros
