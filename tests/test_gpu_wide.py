@@ -20,6 +20,13 @@ CASES = [
     (256, 14336, 4096, 128, 18, True), (256, 4096, 4096, 128, 20, False), (1100, 256, 14340, 128, 16, False),
     (2300, 288, 7172, 32, 16, False), (1024, 256, 16384, 256, 16, False),
 ]
+# small batches on the 32-row tiling: one row tile short, just over and full, k of
+# whole and partial panel blocks, columns short of a block, odd group sizes
+BATCH = [
+    (17, 14336, 4096, 128, 21, True), (32, 4096, 14336, 64, 21, False), (9, 14400, 516, 96, 21, True),
+    (16, 14336, 4, 128, 21, True), (31, 8224, 2052, 32, 21, True), (24, 8192, 8192, 128, 21, True),
+    (25, 4128, 8196, 32, 21, False),
+]
 # N % 4 != 0 (M <= 64 keeps the skinny kernel)
 ODD = [(65, 32, 7, 32), (93, 2080, 1003, 32), (200, 4096, 1001, 64), (129, 160, 1, 32),
        (300, 288, 4098, 96), (700, 640, 2047, 128)]
@@ -49,7 +56,7 @@ def _check(X, qw, s, z, b, G, what):
 
 
 @pytest.mark.parametrize("frac", [False, True])
-@pytest.mark.parametrize("M,K,N,G,cfg,split", CASES)
+@pytest.mark.parametrize("M,K,N,G,cfg,split", CASES + BATCH)
 def test_wide_tilings(M, K, N, G, cfg, split, frac):
     from w4a16 import _lib, w4a16_matmul
 

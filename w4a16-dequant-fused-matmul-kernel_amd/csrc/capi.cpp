@@ -1118,7 +1118,7 @@ int run_planned(const w4a16_plan* p, const void* x, int64_t ldx, const int32_t* 
 }
 
 // ---- automatic calls on the one-wave-per-SIMD prefill kernel (gemm_wide.h) ----
-// Tiling and k-split by a cost model over its five tilings.  A workgroup takes
+// Tiling and k-split by a cost model over its six tilings.  A workgroup takes
 // t0 + panels x tp us (panels of 64 k per wave), a CU holds one, and the time
 // grows with the share of the chip at work (its clock falls: `busy` x share in a
 // single round, a factor `rounds` per round beyond); a split adds its partials'
@@ -1126,7 +1126,8 @@ int run_planned(const w4a16_plan* p, const void* x, int64_t ldx, const int32_t* 
 // 14336, M = 64 .. 4096, G = 128 (us: 256 x 256 tiles 75.4 / 243.5 for 64 / 224
 // panels on 56 / 16 CUs, 94.8 on 224, 104 a round at M = 4096; 128 x 256 49.5 /
 // 157.4, 57.2 on 224; 128 x 128 28.9 / 84.6, 33.1; 64 x 128 22.5 / 69.3, 24.7;
-// 64 x 64 13.7 / 38.0, 15.7).
+// 64 x 64 13.7 / 38.0, 15.7; 32 x 64 at M = 17 11.3 / 29.0 for 64 / 224 panels on
+// 64 CUs, 12.2 on 224, 37 for 128 in two rounds).
 struct WideTiling {
   int cfg, bm, bn, slices;
   double t0, tp, busy, rounds;
@@ -1137,6 +1138,7 @@ constexpr WideTiling kWideTilings[] = {
     {kWide128x128, 128, 128, 2, 6.6, 0.696, 0.12, 1.12},
     {kWide64x128, 64, 128, 2, 3.8, 0.585, 0.07, 1.00},
     {kWide64x64, 64, 64, 4, 4.0, 0.607, 0.17, 1.00},
+    {kWide32x64, 32, 64, 4, 4.2, 0.44, 0.13, 1.06},
 };
 // Half tiles' share of a round (the 256-row tiling's last one).
 constexpr double kWideHalfRound = 0.62;
@@ -1155,6 +1157,7 @@ WideChoice wide_choice(int64_t M, int64_t N, int64_t K, bool any, int cus, size_
   const int64_t panels = (K + 63) / 64;
   for (const WideTiling& t : kWideTilings) {
     if (any && t.cfg == kWide256x256) continue;
+    if (M > 32 && t.cfg == kWide32x64) continue;
     const int64_t tiles = (N + t.bn - 1) / t.bn * ((M + t.bm - 1) / t.bm);
     const int max_split = t.cfg == kWide256x256 ? 1 : 16;
     int last = 0;
@@ -1195,6 +1198,29 @@ bool wide_any(const GemmArgs& a) {
   return !(a.N % 4 == 0 && a.ldy % 4 == 0 && aligned(a.qw, 16) && aligned(a.sc, 8) &&
            aligned(a.zr, 8) && aligned(a.y, 8) && (!a.bias || aligned(a.bias, 8)));
 }
+// Small batches on the 32-row tiling in place of the skinny and 32-row streamed
+// plans: where those are bound by the activations through each CU (all of K for a
+// few columns) or by one wave per SIMD's loads.  Measured on MI355X over M = 5 .. 32
+// x K, N = 2048 .. 28672 x G = 32 / 64 / 128, cold weights (us, those -> this, G =
+// 128): M = 17 / 32, K = 14336, N = 4096 19.6 / 20.0 -> 14.7 / 16.0; N = 2048 18.9 /
+// 19.5 -> 12.0 / 12.7; K = 4096, N = 14336 16.1 / 16.5 -> 12.1 / 12.9; K = 8192, N =
+// 8192 14.9 / 16.6 -> 14.4 / 15.4; M = 9 / 16, K = 14336, N = 4096 15.0 / 16.5 ->
+// 14.8 / 14.8.  Beyond the lines it is slower: M = 32, K = 4096, N = 8192 8.6 -> 11.3
+// (the skinny kernel holds such rows whole); K = 28672, N = 6144 33.9 -> 35.6; K =
+// 14336, N = 28672 59.9 -> 66.3; M = 16, K = 8192, N = 4096 10.7 -> 11.1; N > 8192,
+// unsplit on fewer tiles than CUs: K = 20480, N = 9216, M = 32 35.7 -> 39.5, G = 64,
+// K = 13824, N = 11008 30.8 -> 32.5, G = 32, K = 9728, N = 9216 24.5 -> 27.1, M = 24,
+// K = N = 14336 36.4 -> 36.9.
+bool wide_batch(int64_t M, int64_t N, int64_t K, int64_t G) {
+  if (M < 9 || M > 32 || N < 1 || N % 4 != 0 || G % 32 != 0 || !fits(M, N, K, G)) return false;
+  if (M <= 16) return K >= 14336 && N <= 4096;
+  if (N <= 8192) return K >= 8192 && (K <= 16384 || N <= 4096);
+  if (N > 16384 || K < 4096) return false;
+  const bool wide_groups = G % 64 == 0;
+  return K <= (N <= 12288 ? (wide_groups ? 11008 : 6144) : (wide_groups ? 14336 : 8192)) &&
+         K * N <= 14336 * 14336;
+}
+
 bool scales_zeros_far(const GemmArgs& a) {
   const uintptr_t sc = reinterpret_cast<uintptr_t>(a.sc), zr = reinterpret_cast<uintptr_t>(a.zr);
   const uint64_t dist = sc < zr ? zr - sc : sc - zr;
@@ -1258,10 +1284,18 @@ int run_auto_plan(const w4a16_plan& p, const void* x, int64_t ldx, const int32_t
   const bool ws_ok = ws && aligned(ws, 256);
   const size_t need = p.split_k > 1 ? (size_t)p.workspace_bytes : 0;
   if (x && qw && sc && zr && y && !(p.flags & ~W4A16_PLAN_ANY_ZEROS) &&
-      (need == 0 || (ws_ok && ws_bytes >= need)) && wide_takes(p, a)) {
+      (need == 0 || (ws_ok && ws_bytes >= need))) {
     const int cus = device_cu_count();
     const bool any = wide_any(a);
-    const WideChoice w = wide_choice(M, N, K, any, cus, ws_ok ? ws_bytes : 0);
+    WideChoice w{kWideNone, 1, 0.0};
+    if (wide_takes(p, a)) {
+      w = wide_choice(M, N, K, any, cus, ws_ok ? ws_bytes : 0);
+    } else if (!any && wide_operands_ok(a) && wide_batch(M, N, K, G)) {
+      // (no smaller split for a caller without the workspace: its plan is faster)
+      w = wide_choice(M, N, K, any, cus, kWideWorkspaceMax);
+      if (w.split > 1 && !(ws_ok && ws_bytes >= (size_t)w.split * (size_t)M * (size_t)N * 4u))
+        w.cfg = kWideNone;
+    }
     if (w.cfg != kWideNone)
       return to_status(launch_wide(a, w.cfg, any, w.split, static_cast<float*>(ws), cus,
                                    static_cast<hipStream_t>(stream)));
@@ -1377,7 +1411,8 @@ size_t w4a16_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t group
   // the wide kernel's splits: where the plan is a prefill one it may replace, and
   // where odd widths or alignment send the call to it
   if (group_size % 32 == 0 && M > 0 && N > 0 && K > 0 && fits(M, N, K, group_size) &&
-      (p.kernel == W4A16_KERNEL_MFMA || p.kernel == W4A16_KERNEL_SIMT)) {
+      (p.kernel == W4A16_KERNEL_MFMA || p.kernel == W4A16_KERNEL_SIMT ||
+       wide_batch(M, N, K, group_size))) {
     const WideChoice w = wide_choice(M, N, K, N % 4 != 0, device_cu_count(), kWideWorkspaceMax);
     if (w.split > 1) {
       const size_t need = (size_t)w.split * (size_t)M * (size_t)N * 4u;
@@ -1391,7 +1426,7 @@ int w4a16_gemm_auto_plan(int64_t M, int64_t N, int64_t K, int64_t group_size, w4
   if (int st = w4a16_gemm_plan(M, N, K, group_size, W4A16_KERNEL_AUTO, 0, plan)) return st;
   const bool wide = M > 0 && N > 0 && K > 0 && group_size % 32 == 0 && fits(M, N, K, group_size) &&
                     ((plan->kernel == W4A16_KERNEL_MFMA && M > 32) ||
-                     plan->kernel == W4A16_KERNEL_SIMT);
+                     plan->kernel == W4A16_KERNEL_SIMT || wide_batch(M, N, K, group_size));
   if (!wide) return W4A16_OK;
   const WideChoice w = wide_choice(M, N, K, N % 4 != 0, device_cu_count(),
                                    w4a16_gemm_workspace_bytes(M, N, K, group_size));

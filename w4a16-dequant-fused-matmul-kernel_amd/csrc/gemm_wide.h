@@ -30,6 +30,16 @@
 //     panels ahead (128-byte rows, octet slots XOR-swizzled by (row / 2) % 8: no
 //     bank conflicts), weights, scales and zeros into registers three panels
 //     ahead; one barrier per panel.
+// Tiles of 32 and 64 rows wait on memory, not on the matrix cores: there the
+// activations run three panels ahead and the weights four, and a step's wait
+// leaves in flight all that the two newest steps issued (waiting for all but the
+// last activations drained the weights each panel, a round trip to memory per 64
+// k).  Measured on MI355X, 32 x 64 tiles with four k-slices, M = 17, us: K =
+// 14336, N = 4096 unsplit / split 4 37.8 / 17.1 -> 29.0 / 14.6; K = 4096, N =
+// 14336 14.5 -> 12.2 (a CU's activation lines bound it now: 64 x 64 tiles, twice
+// the lines, gained 0-5 %, taller ones nothing and keep the depth they had).
+// The `any` form holds a column's scale in a register each: joining two as they
+// arrive would wait for each load in turn.
 // kKS = 2 or 4 k-slices per workgroup (waves along K instead of N) serve shapes
 // with few tiles; the slices' sums meet in LDS in slice order.
 // Scales and zeros have a buffer resource each: they may lie anywhere.
@@ -100,6 +110,10 @@ __device__ __forceinline__ void wide_tile(const WideArgs& g, int m0, int n0, int
   constexpr int kAL = kRows / 8;               // its 8-row loads per panel
   static_assert(kRows % 16 == 0, "the swizzle's period");
   constexpr int kPanel = kKS * kBM * 8;
+  // activations' and weights' panels ahead (256-row waves have no registers for more,
+  // 128-row ones gain nothing by it)
+  constexpr bool kDeep = kMT <= 4;
+  constexpr int kXA = kDeep ? 3 : 2, kWA = kDeep ? 4 : 3;
   const int M = g.M, N = g.N, K = g.K;
 
   const int tid = threadIdx.x;
@@ -160,21 +174,34 @@ __device__ __forceinline__ void wide_tile(const WideArgs& g, int m0, int n0, int
   // One panel's words, scales and zeros.  kSZ1: G % 64 == 0, both halves of a
   // panel lie in one group.
   constexpr int kH = kSZ1 ? 1 : 2;
+  // kAny: one column's 16 bits a register (joining two would wait for their loads)
+  using Halves = std::conditional_t<kAny, u32x4, u32x2>;
   struct Panel {
     u32x4 w[2];
-    u32x2 s[kH], z[kH];
+    Halves s[kH], z[kH];
   };
-  auto load_halves = [&](__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) -> u32x2 {
+  // Vector loads of load_w, and what may be in flight where panel kt + 1's
+  // activations must have landed.  Loads retire in order, so three panels ahead
+  // all that steps kt - 1 and kt issued; two ahead step kt's activations.
+  constexpr int kWL = 2 + 2 * kH * (kAny ? kNT : 1);
+  constexpr int kSince = 2 * (kAL + kWL);
+  constexpr int kInFlight = !kDeep ? kAL : kSince < 63 ? kSince : 63;
+  auto load_halves = [&](__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) -> Halves {
     if constexpr (kAny) {
-      uint32_t v[4];
+      Halves v;
 #pragma unroll
-      for (int c = 0; c < 4; ++c)
+      for (int c = 0; c < kNT; ++c)
         v[c] = (uint32_t)(uint16_t)__builtin_amdgcn_raw_buffer_load_b16(
             r, (int)(voff + 2u * (uint32_t)c), (int)soff, 0);
-      return u32x2{v[0] | (v[1] << 16), v[2] | (v[3] << 16)};
+      return v;
     } else {
       return __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(r, (int)voff, (int)soff, 0));
     }
+  };
+  // column c's half, twice
+  auto half2 = [&](const Halves& v, int c) {
+    if constexpr (kAny) return as_h2(__builtin_amdgcn_perm(v[c], v[c], 0x01000100u));
+    else return as_h2(__builtin_amdgcn_perm(v[c / 2], v[c / 2], c & 1 ? 0x03020302u : 0x01000100u));
   };
   auto load_w = [&](int kt, Panel& p) {
     const bool in = kt < KT;
@@ -228,12 +255,10 @@ __device__ __forceinline__ void wide_tile(const WideArgs& g, int m0, int n0, int
   f16x2 dt[2][4], ds[2];       // differences and scales of two columns
   f16x2 pr_s[2], pr_z[2];      // the constants of the next two
   auto prep_s = [&](const Panel& p, int h, int c0, int c) {
-    const uint32_t v = p.s[kSZ1 ? 0 : h][c0 / 2];
-    pr_s[c] = as_h2(__builtin_amdgcn_perm(v, v, c ? 0x03020302u : 0x01000100u));
+    pr_s[c] = half2(p.s[kSZ1 ? 0 : h], c0 + c);
   };
   auto prep_z = [&](const Panel& p, int h, int c0, int c) {
-    const uint32_t v = p.z[kSZ1 ? 0 : h][c0 / 2];
-    const f16x2 z2 = as_h2(__builtin_amdgcn_perm(v, v, c ? 0x03020302u : 0x01000100u));
+    const f16x2 z2 = half2(p.z[kSZ1 ? 0 : h], c0 + c);
     pr_z[c] = AZ ? z2 : z2 + f16x2{(f16)1024.0f, (f16)64.0f};
   };
   auto diff = [&](uint32_t masked, int c) {
@@ -265,9 +290,9 @@ __device__ __forceinline__ void wide_tile(const WideArgs& g, int m0, int n0, int
       asm volatile("s_nop 1");
       __builtin_amdgcn_sched_barrier(0);
       if constexpr (q == 3) {
-        // this wave's activations of panel kt + 1 are there (the kAL loads of
-        // panel kt + 2 since may be in flight); then everyone's of this slice
-        __builtin_amdgcn_s_waitcnt(vmcnt_only(kAL));
+        // this wave's activations of panel kt + 1 are there; then everyone's of
+        // this slice
+        __builtin_amdgcn_s_waitcnt(vmcnt_only(kInFlight));
         if constexpr (kWN > 1) tile_barrier();
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -307,11 +332,13 @@ __device__ __forceinline__ void wide_tile(const WideArgs& g, int m0, int n0, int
           }
         });
         constexpr int kGap = kU >= 4 ? kU / 2 : 1;
-        if constexpr (q == 3 && t == 1) load_w(kt + 3, st[(s + 3) % 4]);
+        // four ahead: into the set of panel kt, whose last words were unpacked in
+        // sub-step 0
+        if constexpr (q == (kDeep ? 1 : 3) && t == 1) load_w(kt + kWA, st[(s + kWA) % 4]);
         if constexpr (q < 3 && t % kGap == 1 % kGap && t / kGap < kLd)
-          load_a(std::integral_constant<int, s + 2>{},
+          load_a(std::integral_constant<int, s + kXA>{},
                  std::integral_constant<int, kAL * q / 3 + t / kGap>{},
-                 std::integral_constant<int, kAL * q / 3 + t / kGap + 1>{}, kt + 2);
+                 std::integral_constant<int, kAL * q / 3 + t / kGap + 1>{}, kt + kXA);
         // the next sub-step's fragments, early: they are there by its start
         if constexpr (t >= 1 && t - 1 < kU) an[t - 1] = read_a(An, (q + 1) / 2 % 2, (q + 1) % 2, t - 1);
         __builtin_amdgcn_sched_barrier(0);
@@ -325,15 +352,31 @@ __device__ __forceinline__ void wide_tile(const WideArgs& g, int m0, int n0, int
   const std::integral_constant<int, 3> c3{};
   const std::integral_constant<int, kAL> call{};
   load_a(c0, c0, call, KS0);
-  load_w(KS0, st[0]);
-  __builtin_amdgcn_sched_barrier(0);
-  load_a(c1, c0, call, KS0 + 1);
-  __builtin_amdgcn_sched_barrier(0);
-  load_w(KS0 + 1, st[1]);
-  load_w(KS0 + 2, st[2]);
-  // the kAL loads of panel KS0 + 1 were issued behind those of panel KS0; the
-  // weights' come later still or are waited for where they are used
-  __builtin_amdgcn_s_waitcnt(vmcnt_only(kAL));
+  if constexpr (kDeep) {
+    // no fewer loads behind each panel's activations than where the steps wait
+    __builtin_amdgcn_sched_barrier(0);
+    load_w(KS0, st[0]);
+    load_w(KS0 + 1, st[1]);
+    __builtin_amdgcn_sched_barrier(0);
+    load_a(c1, c0, call, KS0 + 1);
+    __builtin_amdgcn_sched_barrier(0);
+    load_w(KS0 + 2, st[2]);
+    __builtin_amdgcn_sched_barrier(0);
+    load_a(c2, c0, call, KS0 + 2);
+    __builtin_amdgcn_sched_barrier(0);
+    load_w(KS0 + 3, st[3]);
+    __builtin_amdgcn_sched_barrier(0);
+  } else {
+    load_w(KS0, st[0]);
+    __builtin_amdgcn_sched_barrier(0);
+    load_a(c1, c0, call, KS0 + 1);
+    __builtin_amdgcn_sched_barrier(0);
+    load_w(KS0 + 1, st[1]);
+    load_w(KS0 + 2, st[2]);
+  }
+  // panel KS0's activations (the weights are waited for where they are used): at
+  // least so many loads were issued behind them, wherever the weights' lie
+  __builtin_amdgcn_s_waitcnt(vmcnt_only((kXA - 1) * kAL));
   tile_barrier();
 #pragma unroll
   for (int i = 0; i < kU; ++i) a0[i] = read_a(As0, 0, 0, i);
@@ -363,32 +406,47 @@ __device__ __forceinline__ void wide_tile(const WideArgs& g, int m0, int n0, int
 
   // one trip count for the whole workgroup: every wave reaches every barrier
   const int kend = kKS == 1 ? KT : KS0 + KSL;
-  for (int kt = KS0; kt < kend; kt += 4) {
+  auto four = [&](int kt) {
     step(c0, kt);
     step(c1, kt + 1);
     step(c2, kt + 2);
     step(c3, kt + 3);
+  };
+  if constexpr (kDeep) {
+    // one block, entered at least once (kend > KS0): no load can move to where its
+    // result is used, past a wait that counts it
+    int kt = KS0;
+    do {
+      four(kt);
+      kt += 4;
+    } while (kt < kend);
+  } else {
+    for (int kt = KS0; kt < kend; kt += 4) four(kt);
   }
   // the last MFMAs' results (written by asm the compiler cannot see into)
   asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
   __builtin_amdgcn_sched_barrier(0);
 
-  // kKS slices: each finishes kMT / kKS m-tiles.  The others' sums of them go
-  // through the activation buffers (half a panel buffer per wave), once the
-  // loads in flight (zeros past the range) have landed, and are added in slice
-  // order.
-  static_assert(kMT % kKS == 0, "whole m-tiles per slice");
-  constexpr int kOwn = kMT / kKS;
+  // kKS slices: each finishes kMT / kKS m-tiles, or (fewer m-tiles than slices)
+  // kOwnR of the four rows of one.  The others' sums of them go through the
+  // activation buffers (half a panel buffer per wave), once the loads in flight
+  // (zeros past the range) have landed, and are added in slice order.
+  static_assert(kMT % kKS == 0 || kKS % kMT == 0, "whole m-tiles or rows per slice");
+  constexpr bool kByRow = kMT < kKS;
+  constexpr int kOwn = kByRow ? 1 : kMT / kKS, kOwnR = kByRow ? 4 * kMT / kKS : 4;
+  auto owns = [&](int i) { return kKS == 1 || (kByRow ? slice * kMT / kKS : slice) == i / kOwn; };
+  const int r0 = kByRow ? slice % (kKS / kMT) * kOwnR : 0;
   if constexpr (kKS > 1) {
-    static_assert((kMT - kOwn) * kNT * 64 <= kPanel / 2, "a wave's hand-over fits half a buffer");
+    static_assert((kByRow ? kMT : kMT - kOwn) * kNT * 64 <= kPanel / 2,
+                  "a wave's hand-over fits half a buffer");
     auto region = [&](int w) { return (w < 2 ? As0 : As1) + (w & 1) * (kPanel / 2); };
     __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
     tile_barrier();
     uint4* mine = region(wave);
 #pragma unroll
     for (int i = 0; i < kMT; ++i)
-      if (i / kOwn != slice) {
-        const int at = i < slice * kOwn ? i : i - kOwn;
+      if (kByRow || !owns(i)) {
+        const int at = kByRow || i < slice * kOwn ? i : i - kOwn;
 #pragma unroll
         for (int c = 0; c < kNT; ++c)
           mine[(at * kNT + c) * 64 + lane] = __builtin_bit_cast(uint4, acc[i][c]);
@@ -396,15 +454,15 @@ __device__ __forceinline__ void wide_tile(const WideArgs& g, int m0, int n0, int
     tile_barrier();
 #pragma unroll
     for (int i = 0; i < kMT; ++i)
-      if (i / kOwn == slice) {
+      if (owns(i)) {
 #pragma unroll
         for (int c = 0; c < kNT; ++c) {
           f32x4 v{};
 #pragma unroll
           for (int o = 0; o < kKS; ++o) {
             f32x4 x = acc[i][c];
-            if (o != i / kOwn) {
-              const int at = i < o * kOwn ? i : i - kOwn;
+            if (kByRow || o != i / kOwn) {
+              const int at = kByRow || i < o * kOwn ? i : i - kOwn;
               x = __builtin_bit_cast(f32x4, region(o * kWN + wn)[(at * kNT + c) * 64 + lane]);
             }
             v = o == 0 ? x : v + x;
@@ -421,11 +479,11 @@ __device__ __forceinline__ void wide_tile(const WideArgs& g, int m0, int n0, int
   if (kMT < 16 && g.part) {
 #pragma unroll
     for (int i = 0; i < kMT; ++i)
-      if (kKS == 1 || i / kOwn == slice) {
+      if (owns(i)) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int row = rbase + 16 * i + r;
-          if (row < M) {
+          if (row < M && (!kByRow || (r >= r0 && r < r0 + kOwnR))) {
             float* p = g.part + ((size_t)sp * M + row) * N + ncol;
             if constexpr (kAny) {
 #pragma unroll
@@ -448,11 +506,11 @@ __device__ __forceinline__ void wide_tile(const WideArgs& g, int m0, int n0, int
   }
 #pragma unroll
   for (int i = 0; i < kMT; ++i)
-    if (kKS == 1 || i / kOwn == slice) {
+    if (owns(i)) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int row = rbase + 16 * i + r;
-        if (row < M) {
+        if (row < M && (!kByRow || (r >= r0 && r < r0 + kOwnR))) {
           f16x4 o;
           o.x = f32_to_f16(acc[i][0][r]);
           o.y = f32_to_f16(acc[i][1][r]);

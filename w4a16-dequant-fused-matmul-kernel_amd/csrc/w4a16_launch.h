@@ -116,7 +116,8 @@ enum WideConfig {
   kWide128x256 = 17,
   kWide128x128 = 18,   // two k-slices per workgroup
   kWide64x128 = 19,    // two
-  kWide64x64 = 20      // four
+  kWide64x64 = 20,     // four
+  kWide32x64 = 21      // four; M <= 32
 };
 // 64-k panels per split (whole 4-panel blocks per slice).
 int wide_split_panels(int K, int split, int slices);

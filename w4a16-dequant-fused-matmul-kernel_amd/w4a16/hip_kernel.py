@@ -11,9 +11,10 @@ kernel is chosen inside ``libw4a16.so`` by shape:
 * other M <= 64 on small weights: skinny GEMM on v_mfma_f32_16x16x32_f16, 16
   columns per workgroup over the whole of K;
 * 4 <= M <= 32 on larger weights: the streamed GEMM on MFMA (32-row tiles,
-  split along K where the tiles are few);
+  split along K where the tiles are few), and from M = 9 on long rows or
+  mid-sized weights 32-row tiles of the prefill GEMM below;
 * larger M, any N, and operands less aligned than the kernels above need: the
-  one-wave-per-SIMD prefill GEMM on MFMA (64 to 256-row tiles, k-slices in the
+  one-wave-per-SIMD prefill GEMM on MFMA (32 to 256-row tiles, k-slices in the
   workgroup and splits across workgroups where the tiles are few);
 * what is left (x rows off 16 bytes, operands >= 2 GiB): the sequential-k SIMT
   kernel.
