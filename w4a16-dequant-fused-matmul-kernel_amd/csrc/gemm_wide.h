@@ -80,6 +80,18 @@ __device__ __forceinline__ void static_for(F&& f) {
 constexpr int vmcnt_only(int n) { return (n & 15) | (n >> 4) << 14 | 0x0F70; }
 constexpr int kLgkmcnt0 = 0xC07F;
 
+// No memory access moves across this, in any pass of the compiler (a scheduling
+// barrier holds only the scheduler).
+__device__ __forceinline__ void pin_accesses() { asm volatile("" ::: "memory"); }
+
+// The same pointer, of which the compiler no longer knows that nothing else writes
+// there: loads through a `const __restrict__` argument move across pin_accesses().
+template <class T>
+__device__ __forceinline__ const T* unrestricted(const T* p) {
+  asm volatile("" : "+s"(p));
+  return p;
+}
+
 // This wave's LDS accesses complete, then s_barrier (no wait for the LDS-direct
 // loads in flight, as __syncthreads() would).
 __device__ __forceinline__ void tile_barrier() {
@@ -136,9 +148,12 @@ __device__ __forceinline__ void wide_tile(const WideArgs& g, int m0, int n0, int
   asm volatile("v_mov_b32 %0, 0x54006400" : "=v"(magic_mix));
   const __amdgpu_buffer_rsrc_t rx =
       make_rsrc(g.X, ((uint32_t)(M - 1) * (uint32_t)g.ldx + (uint32_t)K) * 2u);
-  const __amdgpu_buffer_rsrc_t rw = make_rsrc(g.QW, (uint32_t)KP * (uint32_t)N * 4u);
-  const __amdgpu_buffer_rsrc_t rs = make_rsrc(g.SC, (uint32_t)NG * (uint32_t)N * 2u);
-  const __amdgpu_buffer_rsrc_t rz = make_rsrc(g.ZR, (uint32_t)NG * (uint32_t)N * 2u);
+  const __amdgpu_buffer_rsrc_t rw =
+      make_rsrc(kDeep ? unrestricted(g.QW) : g.QW, (uint32_t)KP * (uint32_t)N * 4u);
+  const __amdgpu_buffer_rsrc_t rs =
+      make_rsrc(kDeep ? unrestricted(g.SC) : g.SC, (uint32_t)NG * (uint32_t)N * 2u);
+  const __amdgpu_buffer_rsrc_t rz =
+      make_rsrc(kDeep ? unrestricted(g.ZR) : g.ZR, (uint32_t)NG * (uint32_t)N * 2u);
 
   // Activation stream: wave wn of a slice fills rows kRows wn .. with kAL loads
   // of 8 rows; lane L writes row 8j + L/8, slot L%8, which holds octet
@@ -182,10 +197,16 @@ __device__ __forceinline__ void wide_tile(const WideArgs& g, int m0, int n0, int
   };
   // Vector loads of load_w, and what may be in flight where panel kt + 1's
   // activations must have landed.  Loads retire in order, so three panels ahead
-  // all that steps kt - 1 and kt issued; two ahead step kt's activations.
+  // all that steps kt - 1 and kt issued; two ahead step kt's activations.  The
+  // former counts weights too, which must then be issued where they are written:
+  // pin() keeps them from moving past a wait (they did, to where a loop first uses
+  // them).  LDS-direct loads stay where they are: they write memory.
   constexpr int kWL = 2 + 2 * kH * (kAny ? kNT : 1);
   constexpr int kSince = 2 * (kAL + kWL);
   constexpr int kInFlight = !kDeep ? kAL : kSince < 63 ? kSince : 63;
+  auto pin = [] {
+    if constexpr (kDeep) pin_accesses();
+  };
   auto load_halves = [&](__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) -> Halves {
     if constexpr (kAny) {
       Halves v;
@@ -292,7 +313,9 @@ __device__ __forceinline__ void wide_tile(const WideArgs& g, int m0, int n0, int
       if constexpr (q == 3) {
         // this wave's activations of panel kt + 1 are there; then everyone's of
         // this slice
+        pin();
         __builtin_amdgcn_s_waitcnt(vmcnt_only(kInFlight));
+        pin();
         if constexpr (kWN > 1) tile_barrier();
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -354,18 +377,18 @@ __device__ __forceinline__ void wide_tile(const WideArgs& g, int m0, int n0, int
   load_a(c0, c0, call, KS0);
   if constexpr (kDeep) {
     // no fewer loads behind each panel's activations than where the steps wait
-    __builtin_amdgcn_sched_barrier(0);
+    pin();
     load_w(KS0, st[0]);
     load_w(KS0 + 1, st[1]);
-    __builtin_amdgcn_sched_barrier(0);
+    pin();
     load_a(c1, c0, call, KS0 + 1);
-    __builtin_amdgcn_sched_barrier(0);
+    pin();
     load_w(KS0 + 2, st[2]);
-    __builtin_amdgcn_sched_barrier(0);
+    pin();
     load_a(c2, c0, call, KS0 + 2);
-    __builtin_amdgcn_sched_barrier(0);
+    pin();
     load_w(KS0 + 3, st[3]);
-    __builtin_amdgcn_sched_barrier(0);
+    pin();
   } else {
     load_w(KS0, st[0]);
     __builtin_amdgcn_sched_barrier(0);
@@ -374,9 +397,12 @@ __device__ __forceinline__ void wide_tile(const WideArgs& g, int m0, int n0, int
     load_w(KS0 + 1, st[1]);
     load_w(KS0 + 2, st[2]);
   }
-  // panel KS0's activations (the weights are waited for where they are used): at
-  // least so many loads were issued behind them, wherever the weights' lie
-  __builtin_amdgcn_s_waitcnt(vmcnt_only((kXA - 1) * kAL));
+  // panel KS0's activations (the weights are waited for where they are used): so
+  // many loads were issued behind them (two panels ahead, whether or not the
+  // weights were)
+  constexpr int kSince0 = (kXA - 1) * kAL + (kDeep ? kWA * kWL : 0);
+  __builtin_amdgcn_s_waitcnt(vmcnt_only(kSince0 < 63 ? kSince0 : 63));
+  pin();
   tile_barrier();
 #pragma unroll
   for (int i = 0; i < kU; ++i) a0[i] = read_a(As0, 0, 0, i);
@@ -413,8 +439,8 @@ __device__ __forceinline__ void wide_tile(const WideArgs& g, int m0, int n0, int
     step(c3, kt + 3);
   };
   if constexpr (kDeep) {
-    // one block, entered at least once (kend > KS0): no load can move to where its
-    // result is used, past a wait that counts it
+    // entered at least once (kend > KS0): a guarded loop's entry would copy, and so
+    // wait for, the loads in flight
     int kt = KS0;
     do {
       four(kt);
