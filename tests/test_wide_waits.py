@@ -82,10 +82,15 @@ def _loads_per_panel(key):
     return 16 * mt // wn // 8, 2 + 2 * halves * (4 if any_ else 1)
 
 
+def _deep(key):
+    """Three panels of activations ahead: tiles of at most 64 rows in vector form."""
+    return key[0] <= 4 and not key[6]
+
+
 def _check(key, code):
     """Raises AssertionError where a counted wait covers too little."""
     acts, weights = _loads_per_panel(key)
-    deep = key[0] <= 4
+    deep = _deep(key)
     first, last = _loop(code)
     prologue = [x for _, x in code[:first]]
     body = [x for _, x in code[first:last + 1]]
@@ -137,7 +142,7 @@ def test_a_load_behind_its_wait_is_seen(tmp_path):
         weights = [i for i, (_, x) in enumerate(code) if "buffer_load" in x and " lds" not in x]
         wait = [i + 1 for i in range(first, last) if code[i][1] == "s_nop 1"][3]
         plants = []
-        if key[0] <= 4:   # (the taller tiles wait for activations behind activations)
+        if _deep(key):   # (the others wait for activations behind activations)
             plants += [(max(i for i in weights if i < first), first),
                        (min(i for i in weights if i > first), wait + 1)]
         for load, to in plants:

@@ -39,7 +39,11 @@
 // 14336 14.5 -> 12.2 (a CU's activation lines bound it now: 64 x 64 tiles, twice
 // the lines, gained 0-5 %, taller ones nothing and keep the depth they had).
 // The `any` form holds a column's scale in a register each: joining two as they
-// arrive would wait for each load in turn.
+// arrive would wait for each load in turn.  It is bound by the issue of its two-byte
+// loads, 16 a panel, so it keeps two and three panels ahead: each panel further asks
+// for one more past the end of k.  64 x 64 tiles, three / two ahead, us: M = 93, K =
+// 2080, N = 1003, G = 32 12.9 / 11.5; M = 65, K = N = 1024 10.3 / 8.9; M = 300, K =
+// 2048, N = 2047 14.5 / 12.2; M = 70, K = 28672, N = 1003 25.9 / 22.4.
 // kKS = 2 or 4 k-slices per workgroup (waves along K instead of N) serve shapes
 // with few tiles; the slices' sums meet in LDS in slice order.
 // Scales and zeros have a buffer resource each: they may lie anywhere.
@@ -123,8 +127,9 @@ __device__ __forceinline__ void wide_tile(const WideArgs& g, int m0, int n0, int
   static_assert(kRows % 16 == 0, "the swizzle's period");
   constexpr int kPanel = kKS * kBM * 8;
   // activations' and weights' panels ahead (256-row waves have no registers for more,
-  // 128-row ones gain nothing by it)
-  constexpr bool kDeep = kMT <= 4;
+  // 128-row ones gain nothing by it, and the `any` form's many small loads cost more
+  // than their latency)
+  constexpr bool kDeep = kMT <= 4 && !kAny;
   constexpr int kXA = kDeep ? 3 : 2, kWA = kDeep ? 4 : 3;
   const int M = g.M, N = g.N, K = g.K;
 
