@@ -1156,7 +1156,7 @@ WideChoice wide_choice(int64_t M, int64_t N, int64_t K, bool any, int cus, size_
   WideChoice best{kWideNone, 1, 0.0};
   const int64_t panels = (K + 63) / 64;
   for (const WideTiling& t : kWideTilings) {
-    if (any && t.cfg == kWide256x256) continue;
+    if (any && (t.cfg == kWide256x256 || t.cfg == kWide32x64)) continue;
     if (M > 32 && t.cfg == kWide32x64) continue;
     const int64_t tiles = (N + t.bn - 1) / t.bn * ((M + t.bm - 1) / t.bm);
     const int max_split = t.cfg == kWide256x256 ? 1 : 16;

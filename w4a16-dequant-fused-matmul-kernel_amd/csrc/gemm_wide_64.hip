@@ -24,7 +24,7 @@ hipError_t launch_wide(const GemmArgs& a, int cfg, bool any, int split, float* p
     case kWide128x128: return launch_wide_128x128(a, any, split, part, cus, st);
     case kWide64x128: return launch_wide_tiling<4, false, 2, 2, true>(a, any, split, part, cus, st);
     case kWide64x64: return launch_wide_tiling<4, false, 1, 4, true>(a, any, split, part, cus, st);
-    case kWide32x64: return launch_wide_tiling<2, false, 1, 4, true>(a, any, split, part, cus, st);
+    case kWide32x64: return launch_wide_tiling<2, false, 1, 4, false>(a, any, split, part, cus, st);
     default: return hipErrorInvalidValue;
   }
 }

@@ -108,7 +108,8 @@ hipError_t launch_occ2_gemm(const GemmArgs& a, int split, float* part, hipStream
 
 // One-wave-per-SIMD prefill kernel (gemm_wide.h): tilings of automatic calls
 // only (no plan names them).  `any`: N % 4 != 0 or less alignment than the
-// vector form needs; not on the 256-row tiles.  split > 1: fp32 partials
+// vector form needs; not on the 256-row tiles, nor on the 32-row ones (such calls
+// take the skinny kernel up to M = 64).  split > 1: fp32 partials
 // [split][M][N] in `part`, then the reduction.
 enum WideConfig {
   kWideNone = 0,
