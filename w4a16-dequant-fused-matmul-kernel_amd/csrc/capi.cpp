@@ -1140,6 +1140,32 @@ constexpr WideTiling kWideTilings[] = {
     {kWide64x64, 64, 64, 4, 4.0, 0.607, 0.17, 1.00},
     {kWide32x64, 32, 64, 4, 4.2, 0.44, 0.13, 1.06},
 };
+// What a call was measured to take for a modelled time, us = scale x modelled + add,
+// by G % 64 == 0 or not (whose scales are loaded twice a panel).  Medians over 1700
+// points, M = 33 .. 4096, K, N = 1024 .. 28672, cold weights; one in twenty lies 9 %
+// above it or more, one in twenty 7 % below.
+struct WideActual {
+  int cfg;
+  double scale[2], add[2];
+};
+constexpr WideActual kWideActual[] = {
+    {kWide256x256, {0.97, 1.01}, {-3.0, -2.5}}, {kWide128x256, {1.04, 1.10}, {-3.6, -3.0}},
+    {kWide128x128, {1.10, 1.18}, {-3.0, -3.0}}, {kWide64x128, {1.03, 1.20}, {0.0, -0.5}},
+    {kWide64x64, {0.95, 1.05}, {0.4, 0.4}},
+};
+// The streamed tiles' time (gemm_stream.hip): a CU holds two workgroups.  One alone
+// takes t0 + panels x tp1, and longer by `busy1` x the share of the CUs at work; two
+// t0 + panels x tp2, by `busy2` x the share of the second places taken beyond half;
+// `g32` multiplies the panels' part where G % 64 != 0, a split adds its partials'
+// traffic and `red` each.  Fitted to the same points (within 10 % at 96 % of them).
+struct StreamCost {
+  int cfg;
+  double t0, tp1, busy1, tp2, busy2, g32, red;
+};
+constexpr StreamCost kStreamCosts[] = {
+    {11, 4.2, 0.735, 0.19, 1.43, 0.43, 1.03, 0.03},
+    {13, 4.7, 0.556, 0.235, 1.093, 0.0, 1.05, 0.18},
+};
 // Half tiles' share of a round (the 256-row tiling's last one).
 constexpr double kWideHalfRound = 0.62;
 
@@ -1221,27 +1247,99 @@ bool wide_batch(int64_t M, int64_t N, int64_t K, int64_t G) {
          K * N <= 14336 * 14336;
 }
 
+size_t wide_partials(const WideChoice& w, const GemmArgs& a) {
+  return w.split > 1 ? (size_t)w.split * (size_t)a.M * (size_t)a.N * 4u : 0;
+}
+
 bool scales_zeros_far(const GemmArgs& a) {
   const uintptr_t sc = reinterpret_cast<uintptr_t>(a.sc), zr = reinterpret_cast<uintptr_t>(a.zr);
   const uint64_t dist = sc < zr ? zr - sc : sc - zr;
   return dist + (uint64_t)(a.K / a.G) * (uint64_t)a.N * 2u >= (1ull << 31);
 }
 
-// Whether an automatic call whose plan is `p` (auto_plan's: SIMT where operands
-// are not aligned for the vector kernels) takes the wide kernel: in place of
+// Whether the plan `p` (MFMA, M > 32) is faster than the wide kernel as `w` runs it:
+//   * streamed tiles, by at least 2 %, where the weight is large for a few rows (they
+//     keep two workgroups a CU loading) or the wide tiles leave a round half empty.
+//     Measured on MI355X, cold weights (us, wide -> streamed): M = 57, K = 26624, N =
+//     16896, G = 32 128 -> 82; M = 33, K = 15616, N = 17408, G = 64 65 -> 47; M = 64,
+//     K = N = 28672, G = 128 / 32 158 -> 137 / 193 -> 150; M = 420, K = 14336, N =
+//     8224, G = 32 178 -> 138; M = 4096, K = 14336, N = 2104, G = 32 308 -> 270.  Over
+//     1550 other points the choice is at worst 0.89 of the faster kernel's speed, and
+//     below 0.95 at 9 of them;
+//   * the register-staged tiles of a K of at most three panels, which the wide
+//     kernel's four-panel blocks run past: M = 256, K = 32 / 128, N = 2048 / 5120 7.2 ->
+//     3.6 / 7.4 -> 4.6; M = 3305, K = 128, N = 11008 37.3 -> 22.5; M = 70, K = 192, N =
+//     4096 6.5 -> 5.2 (cfg 2 and 7; the medians are 0.67 of the time at K = 128, 0.80
+//     at 192, 0.92 and 1.0 at 224 and 320); cfg 1 and 6 only to K = 96 (0.9; at 160
+//     1.14).  N < 1024 was not measured.
+// The two-slice tiles (cfg 14), and the register-staged ones of a longer K, were
+// slower at every point.
+bool plan_beats_wide(const w4a16_plan& p, const GemmArgs& a, const WideChoice& w, int cus) {
+  if (a.K <= 192)
+    return a.N >= 1024 && (p.tile_cfg == 2 || p.tile_cfg == 7 || a.K <= 96);
+  const int g32 = a.G % 64 != 0;
+  double wide = w.us;
+  for (const WideActual& t : kWideActual)
+    if (t.cfg == w.cfg) wide = t.scale[g32] * w.us + t.add[g32];
+  for (const StreamCost& c : kStreamCosts) {
+    if (c.cfg != p.tile_cfg) continue;
+    const int64_t whole = (a.K + 63) / 64, panels = (whole + p.split_k - 1) / p.split_k;
+    const int64_t pairs = 2 * (int64_t)cus, full = p.grid_x / pairs;
+    // a few workgroups over fit in where the last splits are shorter than the others
+    const bool fits_in = p.grid_x / p.split_k * whole * 20 <= full * pairs * ((panels + 3) / 4 * 4) * 19;
+    const int64_t rem = full > 0 && fits_in ? 0 : p.grid_x % pairs;
+    const double k = (double)panels * (g32 ? c.g32 : 1.0);
+    auto two = [&](double share) { return (c.t0 + c.tp2 * k) * (1.0 + c.busy2 * (share - 0.5)); };
+    double us = (double)full * two(1.0);
+    if (rem > cus) us += two((double)rem / pairs);
+    else if (rem > 0) us += (c.t0 + c.tp1 * k) * (1.0 + c.busy1 * (double)rem / cus);
+    if (p.split_k > 1)
+      us += 1.8 + c.red * p.split_k + (4.0 * p.split_k + 2.0) * (double)a.M * (double)a.N / 5.0e6;
+    // (below K = 1024 the tiles' ends weigh most and both costs are less sure)
+    return us < (a.K < 1024 ? 0.85 : 0.98) * wide;
+  }
+  return false;
+}
+
+// The wide kernel's tiling and split for an automatic call whose plan is `p`
+// (auto_plan's: SIMT where operands are not aligned for the vector kernels), with
+// partials in `max_bytes`; kWideNone where it is not for this call.  It stands in for
 //   * the streamed and register-tiled prefill kernels from M = 33 (measured on
 //     MI355X against them, us, G = 128: M = 64 / 128 / 256 / 512 / 1024 / 2048 /
 //     4096, K = 4096, N = 14336: 22.3 / 29.8 / 43.4 / 59.8 / 111 / 213 / 404 ->
 //     15.7 / 24.7 / 33.1 / 57.2 / 94.8 / 186 / 362; K = N = 4096, M = 128 / 256 /
 //     512 / 1024 / 4096 20.0 / 25.4 / 32.3 / 45.6 / 119 -> 14.2 / 15.6 / 24.7 /
-//     34.1 / 104), and of the 32-row streamed tiles where scales and zeros lie
-//     too far apart for their one buffer resource;
+//     34.1 / 104; but see plan_beats_wide), and of the 32-row streamed tiles where
+//     scales and zeros lie too far apart for their one buffer resource;
 //   * the SIMT kernel wherever the operands allow it (M = 93, K = 2080, N =
-//     1003, G = 32: 264 -> 27; M = 256, K = 4096, N = 1001 783 -> 41).
-bool wide_takes(const w4a16_plan& p, const GemmArgs& a) {
-  if (!wide_operands_ok(a)) return false;
-  if (p.kernel == W4A16_KERNEL_SIMT) return true;
-  return p.kernel == W4A16_KERNEL_MFMA && (a.M > 32 || (p.tile_cfg >= 11 && scales_zeros_far(a)));
+//     1003, G = 32: 264 -> 11.5; M = 256, K = 4096, N = 1001 783 -> 41);
+//   * small batches (wide_batch), unless its partials do not fit: the plan is faster
+//     than a smaller split.
+WideChoice wide_for(const w4a16_plan& p, const GemmArgs& a, int cus, size_t max_bytes) {
+  const WideChoice none{kWideNone, 1, 0.0};
+  if (!wide_operands_ok(a)) return none;
+  const bool any = wide_any(a);
+  if (p.kernel == W4A16_KERNEL_SIMT ||
+      (p.kernel == W4A16_KERNEL_MFMA && (a.M > 32 || (p.tile_cfg >= 11 && scales_zeros_far(a)))))
+    return wide_choice(a.M, a.N, a.K, any, cus, max_bytes);
+  if (any || !wide_batch(a.M, a.N, a.K, a.G)) return none;
+  const WideChoice w = wide_choice(a.M, a.N, a.K, any, cus, kWideWorkspaceMax);
+  return w.split > 1 && wide_partials(w, a) > max_bytes ? none : w;
+}
+
+// What an automatic call runs: the wide kernel so, or (kWideNone) its plan's.
+WideChoice auto_choice(const w4a16_plan& p, const GemmArgs& a, int cus, size_t max_bytes) {
+  WideChoice w = wide_for(p, a, cus, max_bytes);
+  if (w.cfg != kWideNone && p.kernel == W4A16_KERNEL_MFMA && a.M > 32 && !scales_zeros_far(a) &&
+      plan_beats_wide(p, a, w, cus))
+    w.cfg = kWideNone;
+  return w;
+}
+
+// A shape with aligned, contiguous operands, as the queries ask about it.
+GemmArgs shape_args(int64_t M, int64_t N, int64_t K, int64_t G) {
+  return GemmArgs{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, (int)M, (int)N, (int)K,
+                  (int)G, (int)K, (int)N, false};
 }
 
 // Automatic plan, falling back to the SIMT kernel when the pointers or row
@@ -1286,18 +1384,9 @@ int run_auto_plan(const w4a16_plan& p, const void* x, int64_t ldx, const int32_t
   if (x && qw && sc && zr && y && !(p.flags & ~W4A16_PLAN_ANY_ZEROS) &&
       (need == 0 || (ws_ok && ws_bytes >= need))) {
     const int cus = device_cu_count();
-    const bool any = wide_any(a);
-    WideChoice w{kWideNone, 1, 0.0};
-    if (wide_takes(p, a)) {
-      w = wide_choice(M, N, K, any, cus, ws_ok ? ws_bytes : 0);
-    } else if (!any && wide_operands_ok(a) && wide_batch(M, N, K, G)) {
-      // (no smaller split for a caller without the workspace: its plan is faster)
-      w = wide_choice(M, N, K, any, cus, kWideWorkspaceMax);
-      if (w.split > 1 && !(ws_ok && ws_bytes >= (size_t)w.split * (size_t)M * (size_t)N * 4u))
-        w.cfg = kWideNone;
-    }
+    const WideChoice w = auto_choice(p, a, cus, ws_ok ? ws_bytes : 0);
     if (w.cfg != kWideNone)
-      return to_status(launch_wide(a, w.cfg, any, w.split, static_cast<float*>(ws), cus,
+      return to_status(launch_wide(a, w.cfg, wide_any(a), w.split, static_cast<float*>(ws), cus,
                                    static_cast<hipStream_t>(stream)));
   }
   return run_planned(&p, x, ldx, qw, sc, zr, bias, y, ldy, M, N, K, G, ws, ws_bytes, stream);
@@ -1407,28 +1496,17 @@ size_t w4a16_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t group
   w4a16_plan p;
   if (check_gemm_shape(M, N, K, group_size) != W4A16_OK) return 0;
   if (make_plan(M, N, K, group_size, W4A16_KERNEL_AUTO, 0, &p) != W4A16_OK) return 0;
-  size_t bytes = (size_t)p.workspace_bytes;
-  // the wide kernel's splits: where the plan is a prefill one it may replace, and
-  // where odd widths or alignment send the call to it
-  if (group_size % 32 == 0 && M > 0 && N > 0 && K > 0 && fits(M, N, K, group_size) &&
-      (p.kernel == W4A16_KERNEL_MFMA || p.kernel == W4A16_KERNEL_SIMT ||
-       wide_batch(M, N, K, group_size))) {
-    const WideChoice w = wide_choice(M, N, K, N % 4 != 0, device_cu_count(), kWideWorkspaceMax);
-    if (w.split > 1) {
-      const size_t need = (size_t)w.split * (size_t)M * (size_t)N * 4u;
-      if (need > bytes) bytes = need;
-    }
-  }
-  return bytes;
+  // the plan's, and the wide kernel's where the operands' layout may send a call to
+  // it that this shape's plan would take
+  const GemmArgs a = shape_args(M, N, K, group_size);
+  const WideChoice w = wide_for(p, a, device_cu_count(), kWideWorkspaceMax);
+  return std::max((size_t)p.workspace_bytes, w.cfg != kWideNone ? wide_partials(w, a) : 0);
 }
 
 int w4a16_gemm_auto_plan(int64_t M, int64_t N, int64_t K, int64_t group_size, w4a16_plan* plan) {
   if (int st = w4a16_gemm_plan(M, N, K, group_size, W4A16_KERNEL_AUTO, 0, plan)) return st;
-  const bool wide = M > 0 && N > 0 && K > 0 && group_size % 32 == 0 && fits(M, N, K, group_size) &&
-                    ((plan->kernel == W4A16_KERNEL_MFMA && M > 32) ||
-                     plan->kernel == W4A16_KERNEL_SIMT || wide_batch(M, N, K, group_size));
-  if (!wide) return W4A16_OK;
-  const WideChoice w = wide_choice(M, N, K, N % 4 != 0, device_cu_count(),
+  const GemmArgs a = shape_args(M, N, K, group_size);
+  const WideChoice w = auto_choice(*plan, a, device_cu_count(),
                                    w4a16_gemm_workspace_bytes(M, N, K, group_size));
   for (const WideTiling& t : kWideTilings)
     if (t.cfg == w.cfg) {
@@ -1439,7 +1517,7 @@ int w4a16_gemm_auto_plan(int64_t M, int64_t N, int64_t K, int64_t group_size, w4
       plan->split_k = w.split;
       plan->grid_x = (N + t.bn - 1) / t.bn * ((M + t.bm - 1) / t.bm) * w.split;
       plan->grid_y = 1;
-      plan->workspace_bytes = w.split > 1 ? w.split * M * N * 4 : 0;
+      plan->workspace_bytes = (int64_t)wide_partials(w, a);
     }
   return W4A16_OK;
 }
