@@ -85,8 +85,9 @@ def test_wide_any_width(M, K, N, G, frac):
 @pytest.mark.parametrize("M", [1, 20, 64, 100, 300])
 def test_unaligned_operands(M):
     """Scales, zeros, bias and out off the vector kernels' alignment (views one
-    element into their storage): the skinny kernel up to M = 64, this one beyond;
-    the same bits as their aligned copies on the same kernel family."""
+    element into their storage): the skinny kernel up to M = 64, this one beyond.
+    With scales and zeros off, the same bits wherever the weight, the output and
+    the bias lie."""
     from w4a16 import w4a16_matmul
     from w4a16.hip_kernel import w4a16_linear
 
