@@ -42,6 +42,51 @@ def test_native_module_is_of_these_sources():
     assert mod.gemm(x) is None
 
 
+def test_without_the_native_module(monkeypatch):
+    """A missing or foreign _native.so: one warning, and every call is left to the
+    Python path; an unusable library stays an error."""
+    from w4a16 import _lib, hip_kernel
+
+    def missing(key):
+        raise ImportError("cannot import _native.so")
+
+    class OnDevice(torch.Tensor):
+        is_cuda = True
+
+    loader = hip_kernel._native_gemm
+    x = torch.zeros(2, 64, dtype=torch.float16).as_subclass(OnDevice)
+    monkeypatch.setattr(_lib, "load_native", missing)
+    monkeypatch.setattr(hip_kernel, "_native_gemm", loader)   # undone afterwards
+    with pytest.warns(RuntimeWarning, match="_native.so"):
+        call = hip_kernel._load_native_gemm()
+    assert call(x, x, x, x, None, 32, None, None, None) is None
+    if getattr(loader, "__name__", "") == "_native_gemm":   # not taken the place of yet
+        with pytest.warns(RuntimeWarning, match="_native.so"):
+            assert loader(x, x, x, x, None, 32, None, None, None) is None
+
+    def unusable():
+        raise ImportError("no library")
+
+    monkeypatch.setattr(_lib, "load", unusable)
+    with pytest.raises(ImportError, match="no library"):
+        hip_kernel._load_native_gemm()
+
+
+@pytest.mark.gpu
+def test_calls_without_the_native_module(monkeypatch):
+    """The public entry points on the device with the native call out of the way."""
+    from w4a16 import W4A16Linear, hip_kernel, w4a16_matmul
+
+    x, qw, s, z = _operands(33, 512, 260, 64)
+    lin = torch.nn.Linear(512, 260, device=DEV, dtype=torch.float16)
+    layer = W4A16Linear.from_linear(lin, 64)
+    want = w4a16_matmul(x, qw, s, z, 64), layer(x[None])
+    monkeypatch.setattr(hip_kernel, "_native_gemm", lambda *args: None)
+    log("without the native module")
+    assert torch.equal(w4a16_matmul(x, qw, s, z, 64), want[0])
+    assert torch.equal(layer(x[None]), want[1])
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,K,N,G,frac", [(1, 256, 256, 128, False), (7, 512, 260, 64, True),
                                           (33, 1024, 1003, 32, False), (300, 512, 1024, 128, True),

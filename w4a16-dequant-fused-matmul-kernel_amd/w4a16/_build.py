@@ -105,17 +105,22 @@ def _link(objs: list[str], path: str, verbose: bool) -> None:
 
 NATIVE_SOURCE = "native.cpp"
 NATIVE_PATH = os.path.join(PKG_DIR, "_native.so")
+NATIVE_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1",
+                "-DUSE_ROCM=1"]
+NATIVE_LIBS = ["-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip", "-ldl"]
 
 
 def native_hash() -> str:
     """Like source_hash(), for the CPython module _native.so: its source, the
-    public header, and the torch and Python versions it is compiled against."""
+    public header, the compiler flags, and the torch and Python versions it is
+    compiled against."""
     import torch
 
     h = hashlib.sha256()
     for path in (os.path.join(CSRC, NATIVE_SOURCE), PUBLIC_HEADER):
         with open(path, "rb") as f:
             h.update(f.read())
+    h.update(repr((NATIVE_FLAGS, NATIVE_LIBS)).encode())
     h.update(f"{torch.__version__} {sys.version_info[:2]}".encode())
     return h.hexdigest()
 
@@ -129,9 +134,8 @@ def build_native(verbose: bool = False) -> str:
     root = os.path.dirname(torch.__file__)
     rocm = os.path.dirname(os.path.dirname(os.path.realpath(hipcc())))
     tmp = NATIVE_PATH + ".tmp"
-    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
+    cmd = ["g++", *NATIVE_FLAGS,
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
-           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
            f'-DW4A16_NATIVE_HASH="{native_hash()}"',
            *(f"-isystem{p}" for p in (os.path.join(root, "include"),
                                       os.path.join(root, "include", "torch", "csrc", "api",
@@ -139,7 +143,7 @@ def build_native(verbose: bool = False) -> str:
                                       os.path.join(rocm, "include"), "/opt/rocm/include",
                                       sysconfig.get_paths()["include"])),
            os.path.join(CSRC, NATIVE_SOURCE), "-o", tmp, "-L" + os.path.join(root, "lib"),
-           "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip", "-ldl"]
+           *NATIVE_LIBS]
     if verbose:
         print(" ".join(cmd), flush=True)
     res = subprocess.run(cmd, capture_output=True, text=True)
@@ -151,15 +155,16 @@ def build_native(verbose: bool = False) -> str:
 
 def build(verbose: bool = False, jobs: int | None = None) -> str:
     """Compile every source, link libw4a16.so and compile _native.so; returns the
-    library path."""
+    library path.  Where _native.so does not compile (no g++, no torch headers) the
+    library is there all the same, and the error is raised last."""
     os.makedirs(BUILD_DIR, exist_ok=True)
     jobs = jobs or min(len(SOURCES), os.cpu_count() or 1, 8)
     defines = [f'-DW4A16_SOURCE_HASH="{source_hash()}"']
     with ThreadPoolExecutor(max_workers=jobs) as ex:
         native = ex.submit(build_native, verbose)
         objs = list(ex.map(lambda s: _compile(s, verbose, defines), SOURCES))
+        _link(objs, LIB_PATH, verbose)
         native.result()
-    _link(objs, LIB_PATH, verbose)
     return LIB_PATH
 
 

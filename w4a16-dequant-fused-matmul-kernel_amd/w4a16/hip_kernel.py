@@ -196,16 +196,29 @@ def _output(x: Tensor, M: int, N: int, out: Tensor | None) -> Tensor:
     return out
 
 
+def _load_native_gemm():
+    """The automatic call in one C function (csrc/native.cpp).  Without a module of
+    these sources and this torch every call goes through the checks and the launch
+    below instead: the same kernels and results, 8-15 us more host time a call."""
+    _lib.load()   # an unusable library is an error, as everywhere
+    try:
+        return _lib.load_native(_ZKEY).gemm
+    except ImportError as e:
+        warnings.warn(f"w4a16: {e}; calls are checked and launched from Python meanwhile "
+                      "(the same kernels, 8-15 us more host time each)", RuntimeWarning,
+                      stacklevel=4)
+        return lambda *args: None
+
+
 def _native_gemm(x, *rest):
-    """The automatic call in one C function (csrc/native.cpp): y, or None where
-    the checks and the launch below have to run.  This loads it on the first
-    call with device operands and takes its place."""
+    """The native automatic call: y, or None where the checks and the launch below
+    have to run.  This loads it on the first call with device operands and takes its
+    place."""
     global _native_gemm
     if not (isinstance(x, Tensor) and x.is_cuda):
         return None
-    fn = _lib.load_native(_ZKEY).gemm
-    _native_gemm = fn
-    return fn(x, *rest)
+    _native_gemm = _load_native_gemm()
+    return _native_gemm(x, *rest)
 
 
 def linear_native(x: Tensor, qweight, scales, zeros, bias, group_size: int, in_features: int,
