@@ -193,6 +193,55 @@ def test_quantize_non_finite_raises():
             quantize_weight(W, 32)
 
 
+@pytest.mark.parametrize("transposed", [False, True])
+@pytest.mark.parametrize("N", [8, 261])
+@pytest.mark.parametrize("G", [8, 32, 64, 128, 256, 520])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_quantize_one_non_finite_weight(dtype, G, N, transposed):
+    """One infinity or NaN anywhere raises: one, two and four waves a group, groups
+    read twice, columns together and apart, and a transposed weight read in place
+    (G = 32 .. 256) in a partial 512-k chunk and column tile.  The weight before it,
+    and the one after, quantise."""
+    from w4a16 import quantize_weight
+
+    K = 5 * G
+    log(f"quantize one non-finite G={G} N={N} {dtype} transposed={transposed}")
+    g = torch.Generator().manual_seed(G + N)
+    W = (torch.randn((N, K) if transposed else (K, N), generator=g) * 0.02).to(dtype).to(DEV)
+    W = W.t() if transposed else W
+    quantize_weight(W, G)
+    spots = [(0, 0), (0, N - 1), (K - 1, 0), (K - 1, N - 1), (K - G, N // 2), (K - G // 2, N - 1),
+             (2 * G - 1, 1), (G // 2 + 1, 4)]
+    for i, (k, n) in enumerate(spots):
+        bad = (float("inf"), float("-inf"), float("nan"))[(i + G + N) % 3]
+        keep = W[k, n].clone()
+        W[k, n] = bad
+        with pytest.raises(AssertionError):
+            quantize_weight(W, G)
+        W[k, n] = keep
+    _assert_quant_equal(W, G, f"finite again G={G} N={N}")
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("bad", [float("inf"), float("-inf"), float("nan")])
+def test_from_linear_non_finite_weight(dtype, bad):
+    """from_linear raises what quantize_weight raises, and the next layer is made."""
+    from w4a16 import W4A16Linear
+
+    log(f"from_linear non-finite {bad} {dtype}")
+    lin = torch.nn.Linear(640, 67, device=DEV, dtype=dtype)
+    with torch.no_grad():
+        keep = lin.weight[66, 639].clone()
+        lin.weight[66, 639] = bad
+        with pytest.raises(AssertionError, match="non-finite"):
+            W4A16Linear.from_linear(lin, 128)
+        lin.weight[66, 639] = keep
+    layer = W4A16Linear.from_linear(lin, 128)
+    ref = O.quantize_weight(np_(lin.weight.detach().float() if dtype == torch.bfloat16
+                                else lin.weight).T.copy(), 128)
+    assert np.array_equal(np_(layer.qweight), ref[0])
+
+
 def test_quantize_cpu_input_returns_cpu():
     """CPU input: computed on the GPU, returned on the CPU, same bits."""
     from w4a16 import quantize_weight
