@@ -148,6 +148,24 @@ def test_quantize_ties_and_scales_every_group_split(G, dtype, N):
     _assert_quant_equal(torch.from_numpy(W).to(dtype), G, f"ties G={G} N={N}")
 
 
+@pytest.mark.parametrize("N", [8, 9])
+@pytest.mark.parametrize("G,groups", [(16, 1023), (16, 1027), (24, 1027), (32, 1023), (32, 1027),
+                                      (40, 511), (40, 515), (64, 511), (64, 515)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_quantize_many_groups(G, groups, dtype, N):
+    """Just under and over the number of waves from which a short group is one or two
+    waves' (four groups or two a workgroup, the last one partial), columns together
+    and apart, with zero minima of both signs."""
+    log(f"quantize many groups G={G} groups={groups} N={N} {dtype}")
+    rng = np.random.default_rng(G * groups + N)
+    W = (rng.integers(-8, 9, (G * groups, N)) * 0.25).astype(np.float32)
+    W[:, ::3] = np.abs(W[:, ::3])
+    W = np.where(W == 0, np.where(rng.random(W.shape) < 0.5, -0.0, 0.0), W)
+    W[::7] += rng.standard_normal(W[::7].shape) * 0.01
+    _assert_quant_equal(torch.from_numpy(W.astype(np.float32)).to(dtype), G,
+                        f"many groups G={G} groups={groups} N={N}")
+
+
 @pytest.mark.parametrize("G", [32, 64, 96, 128, 256, 512])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32, torch.bfloat16])
 def test_quantize_transposed_weight(G, dtype):
@@ -349,7 +367,8 @@ def test_dequant_bit_exact(K, N, G):
     assert np.array_equal(np_(out).view(np.uint16), ref.view(np.uint16))
 
 
-@pytest.mark.parametrize("N,off", [(8, 0), (2056, 0), (4, 0), (1028, 0), (2048, 4), (2048, 2), (1027, 0)])
+@pytest.mark.parametrize("N,off", [(8, 0), (2056, 0), (4, 0), (1028, 0), (2048, 4), (2048, 2), (1027, 0),
+                                   (124, 0), (128, 0), (132, 0)])
 @pytest.mark.parametrize("G", [8, 40, 128])
 def test_dequant_columns_per_lane(N, off, G):
     """8, 4 or 1 columns a lane by N and the alignment of scales and zeros (off =

@@ -1271,12 +1271,12 @@ bool scales_zeros_far(const GemmArgs& a) {
 //     3.6 / 7.4 -> 4.6; M = 3305, K = 128, N = 11008 37.3 -> 22.5; M = 70, K = 192, N =
 //     4096 6.5 -> 5.2 (cfg 2 and 7; the medians are 0.67 of the time at K = 128, 0.80
 //     at 192, 0.92 and 1.0 at 224 and 320); cfg 1 and 6 only to K = 96 (0.9; at 160
-//     1.14).  N < 1024 was not measured.
+//     1.14).
 // The two-slice tiles (cfg 14), and the register-staged ones of a longer K, were
 // slower at every point.
 bool plan_beats_wide(const w4a16_plan& p, const GemmArgs& a, const WideChoice& w, int cus) {
   if (a.K <= 192)
-    return a.N >= 1024 && (p.tile_cfg == 2 || p.tile_cfg == 7 || a.K <= 96);
+    return a.N >= 128 && (p.tile_cfg == 2 || p.tile_cfg == 7 || a.K <= 96);
   const int g32 = a.G % 64 != 0;
   double wide = w.us;
   for (const WideActual& t : kWideActual)

@@ -783,11 +783,19 @@ hipError_t quantize_tile_launch(const typename IN::T* w, uint32_t* q, uint16_t* 
   // Waves per group and octets per wave, so that a wave keeps about four
   // octets (32 rows) in registers whatever G: one wave per group up to G = 32,
   // two at 64, four beyond; more than 8 (fp16) / 4 (fp32) octets a wave are
-  // read twice.
+  // read twice.  Where that leaves fewer waves than SIMDs the time is one wave's
+  // own, so its octets go to four waves (G = 32, us, one wave a group -> four: K =
+  // 3712, N = 64 9.2 -> 3.7; K = 768, N = 320 7.6 -> 4.2; at 1024 waves, K = 4096, N =
+  // 2048, 6.2 against 6.9).  So they do with columns apart, whose loads a wave issues
+  // one by one (K = 4096, N = 2045, G = 32 / 64 17.2 / 17.5 -> 11.0 / 11.8; G = 24,
+  // whose three octets leave one of four waves idle, K = 4080, N = 14335 82).
   const int octs = G / 8, per = (octs + 3) / 4;
   constexpr int kMaxKeep = sizeof(typename IN::T) == 2 ? 8 : 4;
-  const int gpb = octs <= 4 ? 4 : octs <= 8 ? 2 : 1;   // groups per workgroup
-  auto k = octs <= 1   ? quantize_tile_kernel<IN, 1, 1, VEC>
+  const int64_t waves = (int64_t)(K / G) * ((N + 255) / 256) * (octs <= 4 ? 1 : 2);
+  const bool four = octs > 1 && octs <= 8 && (waves < 1024 || (!VEC && octs >= 4));
+  const int gpb = four ? 1 : octs <= 4 ? 4 : octs <= 8 ? 2 : 1;   // groups per workgroup
+  auto k = four        ? quantize_tile_kernel<IN, 4, 4, VEC>
+           : octs <= 1 ? quantize_tile_kernel<IN, 1, 1, VEC>
            : octs <= 2 ? quantize_tile_kernel<IN, 2, 1, VEC>
            : octs <= 4 ? quantize_tile_kernel<IN, 4, 1, VEC>
            : octs <= 8 ? quantize_tile_kernel<IN, 4, 2, VEC>
@@ -883,10 +891,12 @@ hipError_t launch_zeros_check(const void* zr, int64_t n, int32_t* flag, hipStrea
 hipError_t launch_dequant(const int32_t* qw, const void* sc, const void* zr, void* w, int K,
                           int N, int G, hipStream_t st) {
   // 8 columns a lane where rows and pointers allow its 16-byte accesses, 4 where
-  // they allow 8-byte ones; else (and where a packed row holds two groups) one
+  // they allow 8-byte ones; else (and where a packed row holds two groups, and on
+  // rows too short to give a wave's lanes several columns each: N = 64, K = 4736 /
+  // 11520 2.5 / 3.0 us at 8 columns, 2.0 / 2.4 at one; N = 128 a tie) one
   auto ok = [&](int c) {
     const uintptr_t m = 2 * (uintptr_t)c - 1;
-    return N % c == 0 && G % 8 == 0 &&
+    return N % c == 0 && N >= 128 && G % 8 == 0 &&
            (((reinterpret_cast<uintptr_t>(sc) | reinterpret_cast<uintptr_t>(zr) |
               reinterpret_cast<uintptr_t>(w)) & m) |
             (reinterpret_cast<uintptr_t>(qw) & 15)) == 0;
