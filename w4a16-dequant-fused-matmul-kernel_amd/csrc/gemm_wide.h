@@ -7,16 +7,14 @@
 //
 // What bounds it: at prefill sizes the chip holds its power limit, so the time
 // follows the energy of a multiply-add and not only the cycles.  Measured on
-// MI355X, M = N = K = 8192, G = 128 (and, same run, hipBLASLt's fp16 product of
-// the dequantised weight at 701 us):
-//   * the two-waves-per-SIMD kernel of 128 x 64 per wave (gemm_stream.hip) 871
-//     us, matrix cores busy 62 % of the cycles at 1.90 GHz;
-//   * this scheme on v_mfma_f32_32x32x16_f16 868 us: 73 % busy, but at 1.65 GHz.
-//     Registers alone, on N(0, 1) data, that instruction sustains 1651 TFLOP/s
-//     and 16x16x32 1916 (both about 2430 on zeros): twice the accumulator
-//     traffic per multiply-add;
-//   * as it stands 754 us = 1458 TFLOP/s (that box: 852 for the first), 72 % busy
-//     at 1.94 GHz.
+// MI355X in one process: registers alone, on N(0, 1) data, v_mfma_f32_16x16x32_f16
+// sustains 1858 TFLOP/s and 32x32x16, with twice the accumulator traffic per
+// multiply-add, 1601 (both about 2345 on zeros); M = N = K = 8192, G = 128:
+//   * the two-waves-per-SIMD kernel of 128 x 64 per wave (gemm_stream.hip) 948 us;
+//   * this kernel 780 us = 1410 TFLOP/s, matrix cores busy 77 % of the cycles;
+//   * hipBLASLt's fp16 product of the dequantised weight 823.
+// (The same scheme first built on 32x32x16 took as long as the streamed kernel: as
+// busy, but at a clock 15 % lower.)
 // Hence:
 //   * a wave owns all rows of the tile and 64 columns (kMT m-tiles x 4 n-tiles),
 //     so every weight is dequantised once per 256 rows (once per 128 rows with
@@ -88,13 +86,10 @@ constexpr int kLgkmcnt0 = 0xC07F;
 // barrier holds only the scheduler).
 __device__ __forceinline__ void pin_accesses() { asm volatile("" ::: "memory"); }
 
-// The same pointer, of which the compiler no longer knows that nothing else writes
-// there: loads through a `const __restrict__` argument move across pin_accesses().
-template <class T>
-__device__ __forceinline__ const T* unrestricted(const T* p) {
-  asm volatile("" : "+s"(p));
-  return p;
-}
+// A read-only argument; kPinned: loads through it stay on their side of
+// pin_accesses() (through a `const __restrict__` one they may move).
+template <class T, bool kPinned>
+using In = std::conditional_t<kPinned, const T*, const T* __restrict__>;
 
 // This wave's LDS accesses complete, then s_barrier (no wait for the LDS-direct
 // loads in flight, as __syncthreads() would).
@@ -114,6 +109,9 @@ struct WideArgs {
   float* part;   // fp32 partials [split][M][N], or nullptr
 };
 
+// Whether a tile keeps three panels of activations and four of weights in flight.
+constexpr bool wide_deep(int mt, bool any) { return mt <= 4 && !any; }
+
 // The tile at (m0, n0) of kBM = 16 kMT rows and kBN = 64 kWN columns, panels
 // [p0, p0 + np) of split sp; As0 .. As3: kKS * kBM * 8 slots each.
 template <int kMT, int kWN, int kKS, bool kSZ1, bool AZ, bool kAny>
@@ -129,7 +127,7 @@ __device__ __forceinline__ void wide_tile(const WideArgs& g, int m0, int n0, int
   // activations' and weights' panels ahead (256-row waves have no registers for more,
   // 128-row ones gain nothing by it, and the `any` form's many small loads cost more
   // than their latency)
-  constexpr bool kDeep = kMT <= 4 && !kAny;
+  constexpr bool kDeep = wide_deep(kMT, kAny);
   constexpr int kXA = kDeep ? 3 : 2, kWA = kDeep ? 4 : 3;
   const int M = g.M, N = g.N, K = g.K;
 
@@ -153,12 +151,9 @@ __device__ __forceinline__ void wide_tile(const WideArgs& g, int m0, int n0, int
   asm volatile("v_mov_b32 %0, 0x54006400" : "=v"(magic_mix));
   const __amdgpu_buffer_rsrc_t rx =
       make_rsrc(g.X, ((uint32_t)(M - 1) * (uint32_t)g.ldx + (uint32_t)K) * 2u);
-  const __amdgpu_buffer_rsrc_t rw =
-      make_rsrc(kDeep ? unrestricted(g.QW) : g.QW, (uint32_t)KP * (uint32_t)N * 4u);
-  const __amdgpu_buffer_rsrc_t rs =
-      make_rsrc(kDeep ? unrestricted(g.SC) : g.SC, (uint32_t)NG * (uint32_t)N * 2u);
-  const __amdgpu_buffer_rsrc_t rz =
-      make_rsrc(kDeep ? unrestricted(g.ZR) : g.ZR, (uint32_t)NG * (uint32_t)N * 2u);
+  const __amdgpu_buffer_rsrc_t rw = make_rsrc(g.QW, (uint32_t)KP * (uint32_t)N * 4u);
+  const __amdgpu_buffer_rsrc_t rs = make_rsrc(g.SC, (uint32_t)NG * (uint32_t)N * 2u);
+  const __amdgpu_buffer_rsrc_t rz = make_rsrc(g.ZR, (uint32_t)NG * (uint32_t)N * 2u);
 
   // Activation stream: wave wn of a slice fills rows kRows wn .. with kAL loads
   // of 8 rows; lane L writes row 8j + L/8, slot L%8, which holds octet
@@ -382,18 +377,22 @@ __device__ __forceinline__ void wide_tile(const WideArgs& g, int m0, int n0, int
   load_a(c0, c0, call, KS0);
   if constexpr (kDeep) {
     // no fewer loads behind each panel's activations than where the steps wait
-    pin();
+    auto next = [&] {
+      pin();
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    next();
     load_w(KS0, st[0]);
     load_w(KS0 + 1, st[1]);
-    pin();
+    next();
     load_a(c1, c0, call, KS0 + 1);
-    pin();
+    next();
     load_w(KS0 + 2, st[2]);
-    pin();
+    next();
     load_a(c2, c0, call, KS0 + 2);
-    pin();
+    next();
     load_w(KS0 + 3, st[3]);
-    pin();
+    next();
   } else {
     load_w(KS0, st[0]);
     __builtin_amdgcn_sched_barrier(0);
@@ -404,8 +403,10 @@ __device__ __forceinline__ void wide_tile(const WideArgs& g, int m0, int n0, int
   }
   // panel KS0's activations (the weights are waited for where they are used): so
   // many loads were issued behind them (two panels ahead, whether or not the
-  // weights were)
-  constexpr int kSince0 = (kXA - 1) * kAL + (kDeep ? kWA * kWL : 0);
+  // weights were).  64-row tiles wait for some of those too: with all of them in
+  // flight the compiler puts waits of its own into the loop, and nothing is gained
+  // (32-row tiles gain, M = 17, K = 14336, N = 4096 13.9 -> 13.4 us).
+  constexpr int kSince0 = (kXA - 1) * kAL + (kMT == 2 ? kWA * kWL : 0);
   __builtin_amdgcn_s_waitcnt(vmcnt_only(kSince0 < 63 ? kSince0 : 63));
   pin();
   tile_barrier();
@@ -574,9 +575,9 @@ __device__ __forceinline__ void wide_tile(const WideArgs& g, int m0, int n0, int
 // preloaded by the dispatch (-amdgpu-kernarg-preload-count).
 template <int kMT, bool kHalf, int kWN, int kKS, bool kSZ1, bool AZ, bool kAny>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
-void wide_kernel(const f16* __restrict__ X, const uint32_t* __restrict__ QW, int M, int N, int K,
-                 int KTS, int ldx, int nb, const uint16_t* __restrict__ SC,
-                 const uint16_t* __restrict__ ZR, uint32_t gmagic, int gshift, int t0, int G,
+void wide_kernel(const f16* __restrict__ X, In<uint32_t, wide_deep(kMT, kAny)> QW, int M, int N,
+                 int K, int KTS, int ldx, int nb, In<uint16_t, wide_deep(kMT, kAny)> SC,
+                 In<uint16_t, wide_deep(kMT, kAny)> ZR, uint32_t gmagic, int gshift, int t0, int G,
                  int ldy, const f16* __restrict__ bias, f16* __restrict__ Y,
                  float* __restrict__ part) {
   constexpr int kBM = 16 * kMT * (kHalf ? 2 : 1), kBN = 16 * kNT * kWN;

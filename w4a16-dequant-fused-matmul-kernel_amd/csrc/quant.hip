@@ -232,8 +232,11 @@ __device__ __forceinline__ bool finite(float v) { return __builtin_fabsf(v) < __
 // Column blocks are the fast grid index: neighbouring workgroups read
 // neighbouring 512-byte (fp16) pieces of the same rows.
 //
-// Bound by memory: about ten VALU instructions a weight, where an IEEE division
-// and an fp32 comparison per weight (about 34) had made it VALU-bound.  Measured
+// About ten VALU instructions a weight, where an IEEE division and an fp32
+// comparison per weight (about 34) had made it VALU-bound; now neither the VALU (57
+// % of the time at K = 4096, N = 14336, G = 128) nor memory (W read once, outputs
+// written once, 22 of 34 us at 6.7 TB/s) bounds it alone: a workgroup loads, reduces
+// and encodes in turn, and those beside it do not fill all of its waits.  Measured
 // on MI355X, K = 4096, N = 14336, us: fp16 G = 128 / 64 / 32 61.2 / 55.7 / 55.3
 // -> 34.0 / 32.9 / 32.8 (4.4-4.7 TB/s of W read and the outputs written; a large
 // copy reaches 5.1), G = 4096 381 -> 171, fp32 G = 128 / 32 68.3 / 53.7 -> 47.4 /
@@ -503,7 +506,8 @@ struct Oct<InF32> {
 // round through LDS (rows padded by a word, no bank conflicts) so that they
 // leave as runs of 32 adjacent words.  A zero minimum takes the sign of the
 // first or last zero in k order (min_step), found from the wave's ballots.
-// Bound by memory.  Measured on MI355X, us, kernel alone: K = 4096, N = 11008 /
+// Bound as quantize_tile_kernel: VALU issue about two thirds of the time, bytes 17
+// of 30 us.  Measured on MI355X, us, kernel alone: K = 4096, N = 11008 /
 // 14336, G = 128 29.9 / 35.2 (4.2 TB/s), fp32 N = 14336 44.8 (6.0 TB/s), K =
 // 8192, N = 28672 116.9; before, a transposing copy (292 at N = 11008) and the
 // row-major quantiser.  16 columns a wave (runs of 64 words, 133 registers, three
