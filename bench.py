@@ -836,8 +836,9 @@ def traffic_from(fetch_csv: str, write_csv: str) -> dict:
     --traffic-probe's counters.  FETCH_SIZE / WRITE_SIZE are in KiB per
     dispatch; each is scaled by what it reads for the calibration copy (the
     probe's first three copy dispatches, 256 MiB read and 256 MiB written
-    each).  A workload's figure is its main kernel's (most dispatched, then
-    longest name); a split-K reduction pass is listed beside it."""
+    each).  bytes_per_launch is the main kernel's (most dispatched, then
+    longest name), bytes_per_call the sum over all kernels of a call (a split-K
+    reduction, a last round's half tiles)."""
     out = {"calibration": {"copy_bytes": 256 << 20}, "kernels": {}}
     for key, path, counter in (("fetch", fetch_csv, "FETCH_SIZE"),
                                ("write", write_csv, "WRITE_SIZE")):
@@ -861,6 +862,8 @@ def traffic_from(fetch_csv: str, write_csv: str) -> dict:
         main = max(e["launches"], key=lambda n: ("reduce" not in n, e["launches"][n]["dispatches"]))
         e["kernel"] = main
         e["bytes_per_launch"] = e["launches"][main]["bytes_per_launch"]
+        e["bytes_per_call"] = sum(k["bytes_per_launch"] * k["dispatches"]
+                                  for k in e["launches"].values()) // e["launches"][main]["dispatches"]
     with open(TRAFFIC_JSON, "w") as f:
         json.dump(out, f, indent=1)
     return out
@@ -931,14 +934,14 @@ def pmc_summary(paths) -> str:
 
 
 def _traffic_for(workload: str):
-    """HBM bytes per launch measured for a workload's kernel (profiles/traffic.json),
+    """HBM bytes per call measured for a workload's kernels (profiles/traffic.json),
     or None when no measurement is recorded."""
     try:
         with open(TRAFFIC_JSON) as f:
             t = json.load(f)
     except (OSError, ValueError):
         return None
-    return t.get("kernels", {}).get(workload, {}).get("bytes_per_launch")
+    return t.get("kernels", {}).get(workload, {}).get("bytes_per_call")
 
 
 def main() -> int:
