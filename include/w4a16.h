@@ -134,18 +134,20 @@ int w4a16_zeros_check_f16(const void* zeros, int64_t count, int32_t* flag, void*
  * What an automatic call (w4a16_gemm_f16, w4a16_linear_f16, w4a16_gemm_f16_auto,
  * and w4a16_gemm_f16_strided without a plan) runs for a shape, given aligned
  * operands and the workspace below.  (w4a16_gemm_f16_noalloc runs
- * w4a16_gemm_plan's.)  Prefill shapes (M > 32), and widths
- * or alignments the planned kernels do not take, run the one-wave-per-SIMD
- * prefill kernel, reported as MFMA tile_cfg 16 .. 20 (256 x 256, 128 x 256, and,
- * with k-slices inside the workgroup, 128 x 128, 64 x 128 and 64 x 64 tiles).
+ * w4a16_gemm_plan's.)  Most prefill shapes (M > 32), widths
+ * and alignments the planned kernels do not take, and some small batches (M = 9
+ * .. 32) run the one-wave-per-SIMD prefill kernel where it is the faster one,
+ * reported as MFMA tile_cfg 16 .. 21 (256 x 256, 128 x 256, and, with k-slices
+ * inside the workgroup, 128 x 128, 64 x 128, 64 x 64 and 32 x 64 tiles).
  * Those numbers only inform: explicit plans name the other kernels
  * (w4a16_gemm_plan) and refuse them.  No reference counterpart.
  */
 int w4a16_gemm_auto_plan(int64_t M, int64_t N, int64_t K, int64_t group_size, w4a16_plan* plan);
 
-/* Workspace bytes an automatic call of this shape can use (0 = none).  Less is
- * enough where w4a16_gemm_plan's workspace_bytes says so: the call then takes
- * fewer k-splits. */
+/* Workspace bytes that cover an automatic call of this shape and its
+ * w4a16_gemm_plan (0 = none); the call may use less, or none.  Less is enough
+ * where w4a16_gemm_plan's workspace_bytes says so: the call then takes fewer
+ * k-splits. */
 size_t w4a16_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t group_size);
 
 /*
