@@ -33,8 +33,8 @@
 // leaves in flight all that the two newest steps issued (waiting for all but the
 // last activations drained the weights each panel, a round trip to memory per 64
 // k).  Measured on MI355X, 32 x 64 tiles with four k-slices, M = 17, us: K =
-// 14336, N = 4096 unsplit / split 4 37.8 / 17.1 -> 29.0 / 14.6; K = 4096, N =
-// 14336 14.5 -> 12.2 (a CU's activation lines bound it now: 64 x 64 tiles, twice
+// 14336, N = 4096 unsplit / split 4 37.8 / 17.1 -> 29.0 / 14.6, 13.4 with the
+// first panel's wait counted as well; K = 4096, N = 14336 14.5 -> 12.2 (a CU's activation lines bound it now: 64 x 64 tiles, twice
 // the lines, gained 0-5 %, taller ones nothing and keep the depth they had).
 // The `any` form holds a column's scale in a register each: joining two as they
 // arrive would wait for each load in turn.  It is bound by the issue of its two-byte
@@ -203,7 +203,7 @@ __device__ __forceinline__ void wide_tile(const WideArgs& g, int m0, int n0, int
   // them).  LDS-direct loads stay where they are: they write memory.
   constexpr int kWL = 2 + 2 * kH * (kAny ? kNT : 1);
   constexpr int kSince = 2 * (kAL + kWL);
-  constexpr int kInFlight = !kDeep ? kAL : kSince < 63 ? kSince : 63;
+  constexpr int kInFlight = kDeep ? kSince : kAL;
   auto pin = [] {
     if constexpr (kDeep) pin_accesses();
   };
@@ -407,7 +407,8 @@ __device__ __forceinline__ void wide_tile(const WideArgs& g, int m0, int n0, int
   // flight the compiler puts waits of its own into the loop, and nothing is gained
   // (32-row tiles gain, M = 17, K = 14336, N = 4096 13.9 -> 13.4 us).
   constexpr int kSince0 = (kXA - 1) * kAL + (kMT == 2 ? kWA * kWL : 0);
-  __builtin_amdgcn_s_waitcnt(vmcnt_only(kSince0 < 63 ? kSince0 : 63));
+  static_assert(kInFlight <= 63 && kSince0 <= 63, "s_waitcnt's counter");
+  __builtin_amdgcn_s_waitcnt(vmcnt_only(kSince0));
   pin();
   tile_barrier();
 #pragma unroll
