@@ -1315,23 +1315,25 @@ bool plan_beats_wide(const w4a16_plan& p, const GemmArgs& a, const WideChoice& w
 //     1003, G = 32: 264 -> 11.5; M = 256, K = 4096, N = 1001 783 -> 41);
 //   * small batches (wide_batch), unless its partials do not fit: the plan is faster
 //     than a smaller split.
-WideChoice wide_for(const w4a16_plan& p, const GemmArgs& a, int cus, size_t max_bytes) {
+WideChoice wide_for(const w4a16_plan& p, const GemmArgs& a, size_t max_bytes) {
   const WideChoice none{kWideNone, 1, 0.0};
-  if (!wide_operands_ok(a)) return none;
+  const bool instead = p.kernel == W4A16_KERNEL_SIMT ||
+                       (p.kernel == W4A16_KERNEL_MFMA &&
+                        (a.M > 32 || (p.tile_cfg >= 11 && scales_zeros_far(a))));
+  // (decode ends here: a call of 5 us, most of it the host's)
+  if ((!instead && !wide_batch(a.M, a.N, a.K, a.G)) || !wide_operands_ok(a)) return none;
   const bool any = wide_any(a);
-  if (p.kernel == W4A16_KERNEL_SIMT ||
-      (p.kernel == W4A16_KERNEL_MFMA && (a.M > 32 || (p.tile_cfg >= 11 && scales_zeros_far(a)))))
-    return wide_choice(a.M, a.N, a.K, any, cus, max_bytes);
-  if (any || !wide_batch(a.M, a.N, a.K, a.G)) return none;
-  const WideChoice w = wide_choice(a.M, a.N, a.K, any, cus, kWideWorkspaceMax);
+  if (instead) return wide_choice(a.M, a.N, a.K, any, device_cu_count(), max_bytes);
+  if (any) return none;
+  const WideChoice w = wide_choice(a.M, a.N, a.K, any, device_cu_count(), kWideWorkspaceMax);
   return w.split > 1 && wide_partials(w, a) > max_bytes ? none : w;
 }
 
 // What an automatic call runs: the wide kernel so, or (kWideNone) its plan's.
-WideChoice auto_choice(const w4a16_plan& p, const GemmArgs& a, int cus, size_t max_bytes) {
-  WideChoice w = wide_for(p, a, cus, max_bytes);
+WideChoice auto_choice(const w4a16_plan& p, const GemmArgs& a, size_t max_bytes) {
+  WideChoice w = wide_for(p, a, max_bytes);
   if (w.cfg != kWideNone && p.kernel == W4A16_KERNEL_MFMA && a.M > 32 && !scales_zeros_far(a) &&
-      plan_beats_wide(p, a, w, cus))
+      plan_beats_wide(p, a, w, device_cu_count()))
     w.cfg = kWideNone;
   return w;
 }
@@ -1383,11 +1385,10 @@ int run_auto_plan(const w4a16_plan& p, const void* x, int64_t ldx, const int32_t
   const size_t need = p.split_k > 1 ? (size_t)p.workspace_bytes : 0;
   if (x && qw && sc && zr && y && !(p.flags & ~W4A16_PLAN_ANY_ZEROS) &&
       (need == 0 || (ws_ok && ws_bytes >= need))) {
-    const int cus = device_cu_count();
-    const WideChoice w = auto_choice(p, a, cus, ws_ok ? ws_bytes : 0);
+    const WideChoice w = auto_choice(p, a, ws_ok ? ws_bytes : 0);
     if (w.cfg != kWideNone)
-      return to_status(launch_wide(a, w.cfg, wide_any(a), w.split, static_cast<float*>(ws), cus,
-                                   static_cast<hipStream_t>(stream)));
+      return to_status(launch_wide(a, w.cfg, wide_any(a), w.split, static_cast<float*>(ws),
+                                   device_cu_count(), static_cast<hipStream_t>(stream)));
   }
   return run_planned(&p, x, ldx, qw, sc, zr, bias, y, ldy, M, N, K, G, ws, ws_bytes, stream);
 }
@@ -1499,15 +1500,14 @@ size_t w4a16_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t group
   // the plan's, and the wide kernel's where the operands' layout may send a call to
   // it that this shape's plan would take
   const GemmArgs a = shape_args(M, N, K, group_size);
-  const WideChoice w = wide_for(p, a, device_cu_count(), kWideWorkspaceMax);
+  const WideChoice w = wide_for(p, a, kWideWorkspaceMax);
   return std::max((size_t)p.workspace_bytes, w.cfg != kWideNone ? wide_partials(w, a) : 0);
 }
 
 int w4a16_gemm_auto_plan(int64_t M, int64_t N, int64_t K, int64_t group_size, w4a16_plan* plan) {
   if (int st = w4a16_gemm_plan(M, N, K, group_size, W4A16_KERNEL_AUTO, 0, plan)) return st;
   const GemmArgs a = shape_args(M, N, K, group_size);
-  const WideChoice w = auto_choice(*plan, a, device_cu_count(),
-                                   w4a16_gemm_workspace_bytes(M, N, K, group_size));
+  const WideChoice w = auto_choice(*plan, a, w4a16_gemm_workspace_bytes(M, N, K, group_size));
   for (const WideTiling& t : kWideTilings)
     if (t.cfg == w.cfg) {
       plan->kernel = W4A16_KERNEL_MFMA;
