@@ -34,6 +34,12 @@ def launched(fn):
             args = re.match(r"I((?:L[a-z]\w*?E)+)E", rest)
             out.append((name, tuple(int(v) for v in re.findall(r"L[a-z](\d+)E", args.group(1)))
                         if args else ()))
+        # a name with no _Float16 in its signature comes demangled
+        m = re.match(r"void w4a16::\(anonymous namespace\)::(\w+)<(.+?)>\(", e.name)
+        if m:
+            vals = (v.strip() for v in m.group(2).split(","))
+            out.append((m.group(1), tuple(int({"true": 1, "false": 0}.get(v, v)) for v in vals
+                                          if re.fullmatch(r"\d+|true|false", v))))
     return out
 
 
@@ -123,3 +129,25 @@ def test_scales_and_zeros_far_apart(M, K, N, G):
     ref = O.reference_w4a16(np_(x), np_(qw[:, cols]), np_(s[:, cols]), np_(z[:, cols]), G)
     assert_gemm_close(far[:, cols], ref, "far apart")
     assert_gemm_close(near[:, cols], ref, "near")
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("G,groups,N,waves", [
+    # octets that fill four waves (4, 7, 8)
+    (32, 1023, 8, 4), (32, 1024, 8, 1), (56, 511, 8, 4), (56, 512, 8, 2), (64, 511, 8, 4), (64, 512, 8, 2),
+    (32, 4095, 9, 4), (32, 4096, 9, 1), (56, 700, 2045, 4), (64, 600, 2045, 4),
+    # and that leave one without (2, 3, 5, 6)
+    (16, 256, 8, 4), (16, 257, 8, 1), (24, 256, 8, 4), (24, 257, 8, 1), (40, 256, 8, 4), (40, 257, 8, 2),
+    (48, 102, 1024, 2), (16, 512, 9, 4), (24, 513, 9, 1), (40, 512, 9, 4), (40, 102, 2045, 2),
+    (48, 513, 9, 2),
+    # and the lengths with one split at every size
+    (8, 2, 9, 1), (72, 2, 9, 4), (128, 2, 8, 4),
+])
+def test_quantise_waves_per_group(G, groups, N, waves, dtype):
+    """Four waves share a short group only where they are all at work or the groups few."""
+    from w4a16 import quantize_weight
+
+    log(f"dispatch quantise G={G} groups={groups} N={N} {dtype}")
+    W = torch.randn(G * groups, N, device=DEV).to(dtype)
+    names = [n for n in launched(lambda: quantize_weight(W, G)) if n[0] == "quantize_tile_kernel"]
+    assert len(names) == 1 and names[0][1][1:] == (waves, int(N % 4 == 0)), names

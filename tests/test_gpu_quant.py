@@ -150,12 +150,13 @@ def test_quantize_ties_and_scales_every_group_split(G, dtype, N):
 
 @pytest.mark.parametrize("N", [8, 9])
 @pytest.mark.parametrize("G,groups", [(16, 1023), (16, 1027), (24, 1027), (32, 1023), (32, 1027),
-                                      (40, 511), (40, 515), (64, 511), (64, 515)])
+                                      (40, 511), (40, 515), (64, 511), (64, 515),
+                                      (16, 255), (24, 257), (48, 513), (32, 4095), (32, 4097)])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
 def test_quantize_many_groups(G, groups, dtype, N):
-    """Just under and over the number of waves from which a short group is one or two
-    waves' (four groups or two a workgroup, the last one partial), columns together
-    and apart, with zero minima of both signs."""
+    """Just under and over the numbers of groups from which a short one is one or two
+    waves' instead of four (four groups or two a workgroup, the last one partial),
+    columns together and apart, with zero minima of both signs."""
     log(f"quantize many groups G={G} groups={groups} N={N} {dtype}")
     rng = np.random.default_rng(G * groups + N)
     W = (rng.integers(-8, 9, (G * groups, N)) * 0.25).astype(np.float32)

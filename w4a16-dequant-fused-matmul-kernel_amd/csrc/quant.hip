@@ -787,16 +787,26 @@ hipError_t quantize_tile_launch(const typename IN::T* w, uint32_t* q, uint16_t* 
   // Waves per group and octets per wave, so that a wave keeps about four
   // octets (32 rows) in registers whatever G: one wave per group up to G = 32,
   // two at 64, four beyond; more than 8 (fp16) / 4 (fp32) octets a wave are
-  // read twice.  Where that leaves fewer waves than SIMDs the time is one wave's
-  // own, so its octets go to four waves (G = 32, us, one wave a group -> four: K =
-  // 3712, N = 64 9.2 -> 3.7; K = 768, N = 320 7.6 -> 4.2; at 1024 waves, K = 4096, N =
-  // 2048, 6.2 against 6.9).  So they do with columns apart, whose loads a wave issues
-  // one by one (K = 4096, N = 2045, G = 32 / 64 17.2 / 17.5 -> 11.0 / 11.8; G = 24,
-  // whose three octets leave one of four waves idle, K = 4080, N = 14335 82).
+  // read twice.  Four waves share a shorter group too where that is faster; `blocks4`
+  // is the number of workgroups it makes.
+  //  * None of the four without an octet (octs 4, 7, 8): below 1024 waves otherwise,
+  //    fewer than SIMDs, where the time is one wave's own (G = 32, us, one wave a
+  //    group -> four: K = 3712, N = 64 9.2 -> 3.7; K = 768, N = 320 7.6 -> 4.2; at 1024
+  //    waves, K = 4096, N = 2048, 6.2 against 6.9).  With columns apart, whose loads a
+  //    wave issues one by one, far beyond (fp16, N = 2045, K = 4096, G = 32 / 64 17.2 /
+  //    17.5 -> 11.0 / 11.8; K = 4096, N = 14335, G = 64 63.8 -> 63.0); at G = 32 up to
+  //    4096 (2688, N = 5121 30.9 -> 28.1; 7616, K = 14336, N = 4098 61.0 against 65.3).
+  //  * Else (octs 2, 3, 5, 6) a wave idles through the workgroup's time: only while
+  //    each CU gets one workgroup (fp16, K = 1000 / 4080, N = 1024, G = 40, 100 / 408
+  //    workgroups 5.1 -> 4.3 / 5.4 against 5.8), with columns apart two (K = 4080,
+  //    N = 1021 / 14335, 408 / 5712 workgroups 12.4 -> 10.9 / 68.6 against 87.2).
   const int octs = G / 8, per = (octs + 3) / 4;
   constexpr int kMaxKeep = sizeof(typename IN::T) == 2 ? 8 : 4;
-  const int64_t waves = (int64_t)(K / G) * ((N + 255) / 256) * (octs <= 4 ? 1 : 2);
-  const bool four = octs > 1 && octs <= 8 && (waves < 1024 || (!VEC && octs >= 4));
+  const int64_t blocks4 = (int64_t)(K / G) * ((N + 255) / 256);
+  const bool four = octs > 1 && octs <= 8 &&
+                    (octs <= 3 * per ? blocks4 <= (VEC ? 256 : 512)
+                     : VEC           ? blocks4 * (octs <= 4 ? 1 : 2) < 1024
+                                     : octs > 4 || blocks4 < 4096);
   const int gpb = four ? 1 : octs <= 4 ? 4 : octs <= 8 ? 2 : 1;   // groups per workgroup
   auto k = four        ? quantize_tile_kernel<IN, 4, 4, VEC>
            : octs <= 1 ? quantize_tile_kernel<IN, 1, 1, VEC>
