@@ -151,3 +151,15 @@ def test_quantise_waves_per_group(G, groups, N, waves, dtype):
     W = torch.randn(G * groups, N, device=DEV).to(dtype)
     names = [n for n in launched(lambda: quantize_weight(W, G)) if n[0] == "quantize_tile_kernel"]
     assert len(names) == 1 and names[0][1][1:] == (waves, int(N % 4 == 0)), names
+
+
+@pytest.mark.parametrize("N,G,columns", [(4, 96, 4), (8, 32, 4), (108, 128, 4), (120, 32, 4), (128, 32, 8),
+                                         (132, 32, 4), (63, 32, 1), (64, 4, 1)])
+def test_dequantise_columns_per_lane(N, G, columns):
+    """Several columns a lane wherever rows allow them, eight from 128 columns."""
+    from w4a16 import dequantize_weight
+
+    log(f"dispatch dequantise N={N} G={G}")
+    _, qw, s, z = operands(1, 384, N, G)
+    names = launched(lambda: dequantize_weight(qw, s, z, G))
+    assert names == [("dequant_vec_kernel", (columns,)) if columns > 1 else ("dequant_kernel", ())], names

@@ -369,7 +369,7 @@ def test_dequant_bit_exact(K, N, G):
 
 
 @pytest.mark.parametrize("N,off", [(8, 0), (2056, 0), (4, 0), (1028, 0), (2048, 4), (2048, 2), (1027, 0),
-                                   (124, 0), (128, 0), (132, 0)])
+                                   (124, 0), (128, 0), (132, 0), (64, 0), (120, 0), (64, 2)])
 @pytest.mark.parametrize("G", [8, 40, 128])
 def test_dequant_columns_per_lane(N, off, G):
     """8, 4 or 1 columns a lane by N and the alignment of scales and zeros (off =

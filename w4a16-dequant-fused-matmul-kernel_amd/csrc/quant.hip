@@ -904,13 +904,14 @@ hipError_t launch_zeros_check(const void* zr, int64_t n, int32_t* flag, hipStrea
 
 hipError_t launch_dequant(const int32_t* qw, const void* sc, const void* zr, void* w, int K,
                           int N, int G, hipStream_t st) {
-  // 8 columns a lane where rows and pointers allow its 16-byte accesses, 4 where
-  // they allow 8-byte ones; else (and where a packed row holds two groups, and on
-  // rows too short to give a wave's lanes several columns each: N = 64, K = 4736 /
-  // 11520 2.5 / 3.0 us at 8 columns, 2.0 / 2.4 at one; N = 128 a tie) one
+  // 8 columns a lane where rows and pointers allow its 16-byte accesses and a row
+  // has 128 columns (N = 64, K = 4736 / 11520 2.5 / 3.0 us at 8 columns, 2.0 / 2.4 at
+  // 4; N = 128 a tie), 4 where they allow 8-byte ones (N = 4, K = 8928 2.2 us against
+  // 2.5 at one; N = 108, K = 4096 2.0 against 2.3); else, and where a packed row holds
+  // two groups, one
   auto ok = [&](int c) {
     const uintptr_t m = 2 * (uintptr_t)c - 1;
-    return N % c == 0 && N >= 128 && G % 8 == 0 &&
+    return N % c == 0 && (c == 4 || N >= 128) && G % 8 == 0 &&
            (((reinterpret_cast<uintptr_t>(sc) | reinterpret_cast<uintptr_t>(zr) |
               reinterpret_cast<uintptr_t>(w)) & m) |
             (reinterpret_cast<uintptr_t>(qw) & 15)) == 0;
